@@ -212,6 +212,37 @@ def test_concurrent_host_threads_on_their_own_streams(torch_gpu):
         assert sorted(ex.map(work, range(4))) == [0, 1, 2, 3]
 
 
+@pytest.mark.parametrize("groups", [1, 2, 31, 32, 33, 64, 65, 128, 129, 257])
+@pytest.mark.parametrize("last", [1, 3, 8])
+def test_spread_launches(torch_gpu, groups, last):
+    """Launches of fewer groups of eight chunks than CUs, whose chunks are dealt
+    over more workgroups (2, 4 or 8 per group, by the group count): group counts on
+    both sides of each line, the last group holding one, three or eight chunks, in
+    one tensor and as a batch that starts with a one-chunk tensor."""
+    import torch
+    from bigsmall_amd.codecs import bf16_chunked as bc
+    from bigsmall_amd.device import ChunkBatch, ChunkJob, StatusWord, upload_bytes
+    rng = np.random.default_rng(groups * 10 + last)
+    n = (8 * (groups - 1) + last) * 1024 - 7                  # 64 lanes x 16 steps; a partial last chunk
+    _say(f"[bsck] spread groups={groups} last={last} n={n}")
+    tensors = [_bf16(rng.standard_normal(n) * 0.02), _bf16(rng.standard_normal(300) * 0.02)]
+    for batch in ([tensors[0]], [tensors[1], tensors[0]]):
+        jobs, outs, keep = [], [], []
+        for w in batch:
+            blob = bc.encode_array(w, steps=16, lanes=64)
+            inf = bc.info(blob)
+            d, o = upload_bytes(blob, "cuda"), torch.zeros(w.size, dtype=torch.int16, device="cuda")
+            jobs.append(ChunkJob(d.data_ptr(), len(blob), o.data_ptr(), w.size, inf.n_chunks, inf.plane_mode))
+            outs.append(o)
+            keep.append(d)
+        st = StatusWord("cuda")
+        ChunkBatch(jobs, "cuda").launch(st)
+        torch.cuda.synchronize()
+        st.check()
+        for w, o in zip(batch, outs):
+            assert o.cpu().numpy().tobytes() == w.tobytes()
+
+
 @pytest.mark.parametrize("mode", [1, 2])
 def test_single_byte_corruptions_decode_or_raise(torch_gpu, mode):
     """Every single-byte corruption of a blob (header, symbol table, chunk
