@@ -1038,10 +1038,6 @@ def main():
                     help="c3 workload: comma-separated subset of studentt,halfzero,fp8_e4m3,fp8_residual")
     ap.add_argument("--ref-codecs", default="",
                     help="reflayer workload: comma-separated subset of bf16_parallel_v1,bf16_se_tans")
-    ap.add_argument("--ref-tables", choices=["auto", "lds", "scalar", "se-scalar", "mant-scalar"], default="auto",
-                    help="refcodecs/reflayer/c3 workloads: where the reference formats' chains read their decode "
-                         "tables (auto: the engine's choice; lds; scalar: SE and mantissa chains through the scalar "
-                         "cache; se-scalar / mant-scalar: only those chains)")
     ap.add_argument("--coder", choices=["rans", "tans"], default="rans",
                     help="layer workload: the engine format's entropy coder (bf16_chunked_v1 or bf16_chunked_tans_v1)")
     ap.add_argument("--engine-only", action="store_true",
@@ -1054,10 +1050,6 @@ def main():
     ap.add_argument("--hbm-probe", action="store_true",
                     help="only measure 2 GiB read-only, write-only and copy streams (HBM rates by direction)")
     args = ap.parse_args()
-    if args.ref_tables != "auto":
-        from bigsmall_amd.codecs import _refstreams
-        _refstreams.RefBatch.SE_SCALAR = args.ref_tables in ("scalar", "se-scalar")   # else False: every SE chain in LDS
-        _refstreams.RefBatch.MANT_SCALAR = args.ref_tables in ("scalar", "mant-scalar")
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one MI355X; multi-GPU runs are not part of it (a model shards by "
               "tensor or layer for decoding, with no exchange between GPUs).", file=sys.stderr)

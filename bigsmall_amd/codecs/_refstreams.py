@@ -31,6 +31,7 @@ from .. import _native
 
 M_SE, M_MANT = 4096, 1024
 SERIAL_MIN_ELEMENTS = 1 << 16   # from here on a wavefront per chain beats a lane per chain
+LANE_CHAINS_MIN = 32            # buckets per mantissa table from which a wavefront decodes 64 of them (csrc/refcodec_decode.hip)
 SE_ALPHABET, MANT_ALPHABET = 512, 128
 
 SE_STREAM_DTYPE = np.dtype([("words", "<u8"), ("x0", "<u4"), ("n_words", "<u4"), ("tail", "<u4"), ("n", "<u4"),
@@ -42,7 +43,7 @@ REF_TASK_DTYPE = np.dtype([("streams", "<u8"), ("se_table", "<u8"), ("bstart", "
                            ("n_streams", "<u4"), ("n_buckets", "<u4"), ("n_tables", "<u4"), ("se_group_begin", "<u4"),
                            ("tile_begin", "<u4"), ("stream_begin", "<u4"), ("mant_group_begin", "<u4"),
                            ("flags", "<u4")])
-# bs_ref_task.flags (include/bigsmall_hip.h)
+# bs_ref_task.flags (include/bigsmall_hip.h): accepted, without effect
 FLAG_SE_SCALAR, FLAG_MANT_SCALAR = 1, 2
 assert SE_STREAM_DTYPE.itemsize == 40 and MANT_BUCKET_DTYPE.itemsize == 40 and REF_TASK_DTYPE.itemsize == 96
 
@@ -111,26 +112,6 @@ def decode_table_se(freqs: np.ndarray) -> np.ndarray:
     out[:, 0] = (freqs[sym] | ((slot - cum[sym]) << 13)).astype(np.uint32)
     out[:, 1] = sym.astype(np.uint32)
     return out
-
-
-def decode_table_se_scalar(freqs: np.ndarray):
-    """The SE table's 4-byte form for a tensor with at most 256 live symbols,
-    none of frequency 4096 (else None): 4096 x {index | f << 8 | (slot - cf)
-    << 20} and the 256 output words (sign << 15 | exponent << 7) of the
-    indexed live symbols, as one uint32 array of 4096 + 256 entries."""
-    freqs = np.asarray(freqs, dtype=np.int64)
-    live = np.flatnonzero(freqs)
-    if len(live) > 256 or freqs.max() >= M_SE:
-        return None
-    index = np.zeros(len(freqs), np.int64)
-    index[live] = np.arange(len(live))
-    sym = np.repeat(np.arange(len(freqs), dtype=np.int64), freqs)
-    cum = np.concatenate([[0], np.cumsum(freqs)[:-1]])
-    slot = np.arange(M_SE, dtype=np.int64)
-    packed = (index[sym] | (freqs[sym] << 8) | ((slot - cum[sym]) << 20)).astype(np.uint32)
-    words = np.zeros(256, np.uint32)
-    words[: len(live)] = (((live >> 8) & 1) << 15) | ((live & 0xFF) << 7)
-    return np.concatenate([packed, words])
 
 
 def decode_table_mant(freqs: np.ndarray) -> np.ndarray:
@@ -336,20 +317,27 @@ def _plan_arrays(plan: RefPlan, blob_ptr: int) -> list[np.ndarray]:
     se = np.zeros(len(plan.se_streams), SE_STREAM_DTYPE)
     for i, (s, first, stride, n) in enumerate(plan.se_streams):
         se[i] = (blob_ptr + s.words_off, s.x0, s.n_words, s.tail, n, first, stride, 0)
-    # buckets longest first: the wave-serial kernel decodes them in groups of
-    # four wavefronts, and a group holds its slot until its longest bucket ends
-    # (every bucket carries its own output position, so the order is free)
+    # every bucket carries its own output position, so the order is free.
+    # Longest first: the wave-serial kernel decodes them in groups of four
+    # wavefronts, and a group holds its slot until its longest bucket ends. With
+    # LANE_CHAINS_MIN buckets per table or more the kernel decodes 64 buckets per
+    # wavefront, which share their table when they are listed table by table (the
+    # tables with the longest buckets first)
     mb = np.zeros(len(plan.buckets), MANT_BUCKET_DTYPE)
-    order = sorted(range(len(plan.buckets)), key=lambda i: -plan.buckets[i][2])
+    size = np.array([b[2] for b in plan.buckets], np.int64)
+    if len(plan.buckets) // LANE_CHAINS_MIN >= max(1, len(plan.mant_freqs)):
+        table = np.array([b[3] for b in plan.buckets], np.int64)
+        longest = np.zeros(len(plan.mant_freqs), np.int64)
+        np.maximum.at(longest, table, size)
+        order = np.lexsort((-size, table, -longest[table])).tolist()
+    else:
+        order = np.argsort(-size, kind="stable").tolist()
     for i, j in enumerate(order):
         s, pb, n, t = plan.buckets[j]
         mb[i] = (blob_ptr + s.words_off, s.x0, s.n_words, s.tail, n, pb, t, 0)
     tables = (np.stack([decode_table_mant(f) for f in plan.mant_freqs]) if plan.mant_freqs
               else np.zeros((1, M_MANT), np.uint32))
     se_table = decode_table_se(plan.se_freqs).reshape(-1)
-    scalar = decode_table_se_scalar(plan.se_freqs)
-    if scalar is not None:                  # the table's 4-byte form follows its pairs (BS_REF_FLAG_SE_SCALAR)
-        se_table = np.concatenate([se_table, scalar])
     return [se.view(np.uint8), se_table.view(np.uint8),
             np.stack(plan.bstart).reshape(-1).view(np.uint8) if plan.bstart else np.zeros(0, np.uint8),
             mb.view(np.uint8), tables.reshape(-1).view(np.uint8)]
@@ -436,17 +424,7 @@ class RefBatch:
     it has completed.
 
     The SE groups are laid out by xcd_bins, so each XCD decodes the SE chains
-    of one tensor or a few. The first tensor of each bin, when it has at most
-    256 live SE symbols, keeps its chains' state in scalar registers and reads
-    a 4-byte table through the scalar cache (a 16 KB table: one per XCD stays
-    resident, where seven tensors' tables spread over every XCD missed, an 8B
-    layer taking 43-45 against 39-41 ms with LDS tables); the other tensors of
-    the bin, and every mantissa chain, read LDS tables (the scalar cache
-    measured no faster for mantissa chains). SE_SCALAR: "auto" (that rule),
-    True (every eligible tensor) or False; MANT_SCALAR: bool."""
-
-    SE_SCALAR = "auto"
-    MANT_SCALAR = False
+    of one tensor or a few."""
 
     def __init__(self, items: list, device):
         import torch
@@ -457,7 +435,7 @@ class RefBatch:
         per = int(L.bs_refcodec_serial_chains_per_group())
         groups = [-(-len(p.se_streams) // per) for p, _, _ in items]
         lens = [max(n for _, _, _, n in p.se_streams) for p, _, _ in items]
-        C, order, begin, first = xcd_bins(groups, lens)
+        C, order, begin, _ = xcd_bins(groups, lens)
         arrays = []
         tasks = np.zeros(len(items), REF_TASK_DTYPE)
         mant_g = tile = stream = work = 0
@@ -467,10 +445,7 @@ class RefBatch:
             ns, nb = len(plan.se_streams), len(plan.buckets)
             nt = max(1, len(plan.mant_freqs))
             tiles = int(L.bs_refcodec_serial_tiles(plan.n, ns))
-            flags = FLAG_MANT_SCALAR if self.MANT_SCALAR else 0
-            if arrays[-4].nbytes > 8 * M_SE and (self.SE_SCALAR is True or (self.SE_SCALAR == "auto" and first[it])):
-                flags |= FLAG_SE_SCALAR        # the SE table carries its 4-byte form
-            tasks[i] = (0, 0, 0, 0, 0, out_ptr, plan.n, work, ns, nb, nt, begin[it], tile, stream, mant_g, flags)
+            tasks[i] = (0, 0, 0, 0, 0, out_ptr, plan.n, work, ns, nb, nt, begin[it], tile, stream, mant_g, 0)
             work += (int(L.bs_refcodec_serial_work_bytes(plan.n, ns)) + 255) & ~255
             mant_g += -(-nb // per)
             tile, stream = tile + ns * tiles, stream + ns
@@ -590,4 +565,4 @@ def decode_host(codec: str, blob: bytes, n_weights: int) -> bytes:
 
 
 __all__ = ["PARSERS", "RefBatch", "RefLaunch", "RefPlan", "serial_ok", "decode_host", "encode_host", "parse_parallel", "parse_tans",
-           "parse_single_kernel", "decode_table_se", "decode_table_se_scalar", "decode_table_mant"]
+           "parse_single_kernel", "decode_table_se", "decode_table_mant"]

@@ -26,6 +26,8 @@
 // exponent, up to 256 of them) are read through the caches.
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "simt.h"
 
 #include "../../include/bigsmall_hip.h"
@@ -135,18 +137,15 @@ __global__ __launch_bounds__(kMantThreads) void mant_kernel(const bs_mant_bucket
 }
 
 // ---- wave-serial path: every SE stream (one for bf16_se_tans and
-// bf16_se_single_kernel, N interleaved ones for bf16_parallel_v1) and every
-// mantissa bucket is a chain decoded by its own wavefront.
+// bf16_se_single_kernel, N interleaved ones for bf16_parallel_v1) is a chain
+// decoded by its own wavefront, and so is every mantissa bucket unless many
+// buckets share a table (lane_chains, below).
 //
-// Each chain is decoded by one wavefront. The chain itself is uniform (every
-// lane computes the same state; the compiler keeps it in scalar registers),
-// the decode table sits in LDS, and the lanes cooperate on everything around
-// it: they load the word stream 1 KB at a time into an LDS byte ring one
-// segment ahead of use, hold a 128-word window of it in two registers (lane
-// l: words base + l and base + 64 + l, moved on at most once per 64 steps) so
-// that a renormalisation takes its word with a readlane and no branch, and
-// they stage 64 consecutive outputs (lane j keeps step j) for one coalesced
-// store. The SE chain writes sign<<15 | exp<<7 of
+// A wavefront's chain keeps its state in a scalar register and its symbols
+// spread over the lanes (serial_chain); the lanes also load the word stream 1 KB
+// at a time into an LDS byte ring one segment ahead of use, hold a 64-word
+// window of it, and keep the symbols of 64 steps (lane j: step j) for one
+// coalesced store. The SE chain writes sign<<15 | exp<<7 of
 // every element and counts the exponents of each tile of kTile symbols of its
 // stream; the mantissa chains, which do not depend on it, run at the same time
 // in other workgroups and write their bucket's mantissas in bucket order. Two
@@ -202,7 +201,7 @@ __device__ __forceinline__ bool stream_ok(const bs_se_stream& S, uint64_t max_le
 // n_streams elements (1.6 of 39 ms for an 8B layer in bf16_parallel_v1).
 __device__ __forceinline__ void tile_count(LDS uint32_t* hist, GLB uint32_t* ghist, uint32_t word, uint32_t lane,
                                            uint32_t i0, uint32_t cnt, uint32_t n) {
-  if (lane < cnt) BS_LDS_ADD(hist + ((word >> 7) & 0xFFu), 1u);
+  if (cnt == (uint32_t)kWave || lane < cnt) BS_LDS_ADD(hist + ((word >> 7) & 0xFFu), 1u);
   const uint32_t end = i0 + cnt;
   if (end % kTile == 0 || end == n) {
     wave_sync();
@@ -224,14 +223,26 @@ __device__ __forceinline__ void tile_count_end(GLB uint32_t* ghist, uint32_t lan
   for (uint64_t i = ((uint64_t)n + kTile - 1) / kTile * 256u + lane; i < (uint64_t)tps * 256u; i += kWave) ghist[i] = 0;
 }
 
-// Decode one chain of n symbols. The LDS table has one 16-byte entry per slot,
-// {f, slot - cf, output, 0} (SE: M = 4096, output the word sign<<15 | exp<<7,
-// stored as u16; mantissa: M = 1024, output one byte per symbol), so a step is
-// one table read and one v_mad_u32_u24 on the state, which every lane holds.
-// One wavefront issues about one instruction per four cycles, so the step is
-// kept to a dozen instructions: the renormalisation is a scalar branch on the
-// state, its word comes from a register window by readlane, and the output is
-// staged with a lane select.
+// Decode one chain of n symbols with the symbols spread over the lanes: lane l
+// holds symbols l*R .. l*R + R-1 (in slot order: f and cf of each), and no table
+// is read. A step forms in every lane the state its symbol would give,
+//   c = f * (x >> log2 M) + (x mod M) - cf  =  x - cf - (M - f) * (x >> log2 M),
+// and that state renormalised with the chain's next word; the one lane whose
+// interval [cf, cf + sum of its f) holds the slot is found by a ballot, and a
+// readlane takes its state as the wave's next (x is uniform, in a scalar
+// register). The interval test runs on the slot shifted to the top of the word
+// (x << (32 - log2 M)), so it needs no mask and covers f = M.
+//
+// What bounds it: one wavefront's in-order issue (about 4.2 cycles per
+// instruction, 8.3 where one uses the last one's result, about 21 from a vector
+// instruction that writes a scalar register to the next scalar instruction),
+// since a chain is serial by its format. Hence no branch in the step (34 cycles
+// taken, 20 not taken, and a renormalisation every sixth step behind it) and no
+// table read (a scalar load through its cache 60 cycles and more, an LDS read 56).
+// MI355X, ns per step with everything around it: 31 with at most 64 symbols (54-57
+// with a table in the scalar cache, 68-77 with one in LDS). A layer of 2048 x 5632
+// in bf16_parallel_v1 5.49 -> 3.48 ms, 4096 x 14336 27.7 -> 17.7 ms, a layer of
+// 512 x 1408 in bf16_se_tans 41.1 -> 22.5 ms (the lane-wise mantissas included).
 //
 // Renormalisation: the reference loops `while x < L and words remain`. From a
 // state x >= L one decode step leaves x >= 2^4 (SE) or 2^6 (mantissa), so one
@@ -239,16 +250,60 @@ __device__ __forceinline__ void tile_count_end(GLB uint32_t* ghist, uint32_t lan
 // and an initial state below L, which no encoder writes, is reported as a
 // corrupt stream. A corrupt stream that runs out of words shifts in its tail
 // word (zero when it has none) and fails the end-of-stream check.
-template <bool SE>
+__device__ __forceinline__ uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t uni64(uint64_t v) {
+  return (uint64_t)uni32((uint32_t)v) | ((uint64_t)uni32((uint32_t)(v >> 32)) << 32);
+}
+
+// A symbol of a chain's table in LDS: f | cf << 16, and its output (SE: the
+// word sign<<15 | exp<<7; mantissa: the 7 bits).
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// This lane's symbols, from the list in LDS (`live` of them, in slot order).
+template <int R, bool SE>
+struct LaneSyms {
+  int32_t nf[R];         // f - M
+  uint32_t cf[R];
+  uint32_t first;        // -(cf of the first) << (32 - log2 M)
+  uint32_t last;         // (the lane's slots << (32 - log2 M)) - 1: the interval test's bound
+  uint32_t bound[R];     // states below this renormalise: the symbol's decode is below L for x < the encode of L
+  uint32_t begin[R];     // (cf - first cf) << (32 - log2 M) of symbols 1 .. R-1
+  __device__ __forceinline__ void load(const LDS u32x2* syms, uint32_t live, uint32_t lane) {
+    constexpr uint32_t kM = SE ? 4096u : 1024u, kTop = SE ? 20u : 22u;
+    uint32_t slots = 0, cf0 = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t i = lane * R + r;
+      const uint32_t e = syms[min(i, live - 1u)].x;
+      const uint32_t f = i < live ? e & 0xFFFFu : 0u;
+      cf[r] = e >> 16;
+      nf[r] = (int32_t)f - (int32_t)kM;
+      bound[r] = f ? ((kL / f) << (32u - kTop)) + kL % f + cf[r] : 0u;
+      if (r == 0) cf0 = cf[0];
+      // an absent symbol begins where no slot is (a shifted slot has zero low bits)
+      begin[r] = i < live ? (cf[r] - cf0) << kTop : 0xFFFFFFFFu;
+      slots += f;
+    }
+    // a lane without symbols matches no slot: its shifted slot is odd, its bound zero
+    first = slots ? 0u - (cf0 << kTop) : 1u;
+    last = slots ? (slots << kTop) - 1u : 0u;
+  }
+};
+
+template <int R, bool SE>
 __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t n_words, uint32_t tail, uint32_t x0,
-                                             uint32_t n, const LDS u32x4* __restrict__ tbl,
-                                             LDS uint8_t* ring, LDS uint16_t* stage, GLB uint8_t* __restrict__ out,
-                                             uint32_t stride, LDS uint32_t* hist, GLB uint32_t* ghist, uint32_t tps,
-                                             int32_t* status) {
-  constexpr uint32_t kSlotMask = SE ? 4095u : 1023u;
-  constexpr uint32_t kShift = SE ? 12u : 10u;
+                                             uint32_t n, const LDS u32x2* syms, uint32_t live, LDS uint8_t* ring,
+                                             GLB uint8_t* __restrict__ out, uint32_t stride, LDS uint32_t* hist,
+                                             GLB uint32_t* ghist, uint32_t tps, int32_t* status) {
+  constexpr uint32_t kLog = SE ? 12u : 10u, kTop = 32u - kLog;
+  constexpr uint32_t kHalf = 32;       // steps between looks at the word window
+  // the descriptor's fields are the same in every lane: say so, so that the
+  // chain's state and word position stay scalar
+  n_words = uni32(n_words);
+  tail = uni32(tail);
+  n = uni32(n);
   const uint32_t lane = __lane_id();
-  const uint64_t wa = (uint64_t)words;
+  const uint64_t wa = uni64((uint64_t)words);
   const GLB uint8_t* A = (const GLB uint8_t*)(wa & ~15ull);
   const uint32_t s_off = (uint32_t)(wa & 15u);
   const uint64_t e_off = s_off + 2ull * n_words;
@@ -257,175 +312,28 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
   uint64_t landed = 0;        // stream bytes [.., landed) are in the ring (relative to A)
   bool inflight = false;      // segment `landed / kSegB` is being loaded into `seg`
   u32x4 seg = {0u, 0u, 0u, 0u};
-  uint32_t x = x0, pos = 0;
-  // Word window: lane l of w_lo / w_hi holds word base + l / base + 64 + l.
-  // At a batch start pos - base < 64, so the batch's at most 64 words are in it.
-  uint32_t base = 0, w_lo = 0, w_hi = 0;
-  if (x0 < kL) {
-    if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
-    return;
-  }
-  if (SE) tile_count_begin(hist, lane);
-  auto ring_word = [&](uint32_t idx) {
-    const uint32_t b = s_off + 2u * idx;
-    return (uint32_t)ring[b & (kRingB - 1u)] | ((uint32_t)ring[(b + 1u) & (kRingB - 1u)] << 8);
-  };
-  // The state stays in a vector register (the empty asm hides its uniformity,
-  // which would otherwise move the update to scalar instructions plus two
-  // readfirstlanes); only the renormalisation test reads it back.
-  BS_OPAQUE(x);
-  auto step = [&](uint32_t j) {
-    const u32x4 e = tbl[x & kSlotMask];
-    uint32_t xn = __umul24(e.x, x >> kShift) + e.y;         // v_mad_u32_u24 (f <= 4096)
-    if ((uint32_t)__builtin_amdgcn_readfirstlane((int)xn) < kL) {   // uniform: a scalar branch
-      const uint32_t d = pos - base;                       // < 128
-      const uint32_t w_a = __builtin_amdgcn_readlane(w_lo, d & 63u);
-      const uint32_t w_b = __builtin_amdgcn_readlane(w_hi, d & 63u);
-      uint32_t w = d < (uint32_t)kWave ? w_a : w_b;
-      w = pos < n_words ? w : tail_word;
-      xn = (xn << 16) | w;
-      ++pos;
-    }
-    x = xn;
-    BS_OPAQUE(x);
-    // the step's output goes to slot j of the wave's 64-entry stage (every
-    // lane writes the same value), read back by lane j after the batch: a
-    // select per step (keep = lane == j ? out : keep) made the optimiser hold
-    // the batch's 64 outputs, or its 64 lane masks, in registers
-    *(volatile LDS uint16_t*)(stage + j) = (uint16_t)e.z;
-  };
-  for (uint32_t i0 = 0; i0 < n; i0 += kWave) {
-    // ring upkeep: the window reaches at most 128 words (256 bytes) past pos
-    const uint64_t consumed = s_off + 2ull * pos;
-    if (inflight) {
-      seg_land(ring, landed / kSegB, lane, seg);
-      landed += kSegB;
-      inflight = false;
-    }
-    while (landed < e_off && landed < consumed + 4u * kWave + 2u) {
-      seg_land(ring, landed / kSegB, lane, seg_block(A, landed / kSegB, lane, s_off, e_off));
-      landed += kSegB;
-    }
-    if (landed < e_off && landed + kSegB <= consumed + kRingB) {
-      seg = seg_block(A, landed / kSegB, lane, s_off, e_off);
-      inflight = true;
-    }
-    wave_sync();
-    if (i0 == 0) {
-      w_lo = ring_word(lane);
-      w_hi = ring_word(kWave + lane);
-    } else if (pos - base >= (uint32_t)kWave) {           // one move keeps pos - base < 64
-      base += kWave;
-      w_lo = w_hi;
-      w_hi = ring_word(base + kWave + lane);
-    }
-    const uint32_t cnt = min((uint32_t)kWave, n - i0);
-    if (cnt == (uint32_t)kWave) {
-#pragma unroll
-      for (uint32_t j = 0; j < (uint32_t)kWave; ++j) step(j);
-    } else {
-      for (uint32_t j = 0; j < cnt; ++j) step(j);
-    }
-    wave_sync();
-    const uint32_t keep = stage[lane];
-    if (lane < cnt) {
-      if (SE) ((GLB uint16_t*)out)[(uint64_t)(i0 + lane) * stride] = (uint16_t)keep;
-      else out[i0 + lane] = (uint8_t)keep;
-    }
-    if (SE) tile_count(hist, ghist, keep, lane, i0, cnt, n);
-  }
-  if (SE) tile_count_end(ghist, lane, n, tps);
-  if (__builtin_amdgcn_readfirstlane(x) != kL || pos != n_eff) {
-    if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
-  }
-}
-
-// The same chain with the state in scalar registers and the table read
-// through the scalar cache (uniform loads, read-only): one s_load_dword and
-// the update in SALU instructions; the step's output goes into one lane of a
-// register. Tables of 4-byte entries: SE, {index | f << 8 | (slot - cf)
-// << 20} (the 16 KB table of a tensor with at most 256 live sign/exponent
-// symbols, none of frequency 4096; the index selects the output word from
-// `out_words`, a 256-entry LDS map applied once per 64 outputs); mantissa,
-// the global table itself {f | (slot - cf) << 11 | symbol << 21} (4 KB per
-// bucket table). A scalar-cache hit comes back sooner than the LDS round
-// trip, and the step issues fewer instructions (C0 in bf16_se_tans: 1.04
-// against 1.22 s on one chain, before the register output). A 16 KB table
-// stays in the scalar cache only while it has the cache of its CUs to
-// itself (an 8B layer in bf16_parallel_v1, every tensor's SE groups spread
-// over every XCD: 43-45 against 39-41 ms with LDS tables), so the host sets
-// it per task and lays the SE groups out by XCD.
-__device__ __forceinline__ uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ uint64_t uni64(uint64_t v) {
-  return (uint64_t)uni32((uint32_t)v) | ((uint64_t)uni32((uint32_t)(v >> 32)) << 32);
-}
-
-template <bool SE>
-__device__ __forceinline__ void serial_chain_scalar(const GLB uint8_t* words, uint32_t n_words, uint32_t tail,
-                                                    uint32_t x0, uint32_t n, const CST uint32_t* t4_in,
-                                                    const LDS uint32_t* out_words, LDS uint8_t* ring,
-                                                    GLB uint8_t* __restrict__ out, uint32_t stride,
-                                                    LDS uint32_t* hist, GLB uint32_t* ghist, uint32_t tps,
-                                                    int32_t* status) {
-  // the descriptor's fields are the same in every lane: say so, so that the
-  // whole chain (state, word position, table address) stays scalar
-  n_words = uni32(n_words);
-  tail = uni32(tail);
-  n = uni32(n);
-  const CST uint32_t* __restrict__ t4 = (const CST uint32_t*)uni64((uint64_t)t4_in);
-  constexpr uint32_t kSlotMask = SE ? 4095u : 1023u;
-  constexpr uint32_t kShift = SE ? 12u : 10u;
-  const uint32_t lane = __lane_id();
-  const uint64_t wa = (uint64_t)words;
-  const GLB uint8_t* A = (const GLB uint8_t*)(wa & ~15ull);
-  const uint32_t s_off = (uint32_t)(wa & 15u);
-  const uint64_t e_off = s_off + 2ull * n_words;
-  const uint32_t n_eff = n_words + ((tail >> 16) & 1u);
-  const uint32_t tail_word = tail & 0xFFFFu;
-  uint64_t landed = 0;
-  bool inflight = false;
-  u32x4 seg = {0u, 0u, 0u, 0u};
-  uint32_t x = __builtin_amdgcn_readfirstlane(x0), pos = 0;
-  uint32_t base = 0, w_lo = 0, w_hi = 0;
+  uint32_t x = uni32(x0);
   if (x < kL) {
     if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
     return;
   }
   if (SE) tile_count_begin(hist, lane);
-  auto ring_word = [&](uint32_t idx) {
-    const uint32_t b = s_off + 2u * idx;
-    return (uint32_t)ring[b & (kRingB - 1u)] | ((uint32_t)ring[(b + 1u) & (kRingB - 1u)] << 8);
-  };
-  uint32_t acc = 0;            // lane j: output j of the batch
-  auto step = [&]() -> uint32_t {
-    const uint32_t e = t4[x & kSlotMask];                  // s_load_dword: x is wave-uniform
-    const uint32_t f = SE ? (e >> 8) & 0xFFFu : e & 0x7FFu;
-    const uint32_t bias = SE ? e >> 20 : (e >> 11) & 0x3FFu;
-    uint32_t xn = f * (x >> kShift) + bias;
-    // uniform: a scalar branch, taken by about one step in five, so laid out
-    // off the straight path
-    if (__builtin_expect(xn < kL, 0)) {
-      const uint32_t d = pos - base;                       // < 128
-      const uint32_t w_a = __builtin_amdgcn_readlane(w_lo, d & 63u);
-      const uint32_t w_b = __builtin_amdgcn_readlane(w_hi, d & 63u);
-      uint32_t w = d < (uint32_t)kWave ? w_a : w_b;
-      w = pos < n_words ? w : tail_word;
-      xn = (xn << 16) | w;
-      ++pos;
-    }
-    x = xn;
-    // the SE index is the entry's low byte, kept as it is
-    return SE ? e : (e >> 21) & 0x7Fu;
-  };
-  for (uint32_t i0 = 0; i0 < n; i0 += kWave) {
-    // ring upkeep: the window reaches at most 128 words (256 bytes) past pos
-    const uint64_t consumed = s_off + 2ull * pos;
+  LaneSyms<R, SE> S;
+  S.load(syms, live, lane);
+  // Word window: lane l of `win` holds word base + l (past the stream: the tail
+  // word); the next word is lane `at`'s. A step takes at most one word, so a
+  // window moved on when `at` has reached kHalf lasts another kHalf steps.
+  uint32_t base = 0, at = kWave, win = 0;
+  auto window = [&]() {
+    base = uni32(base + (at == kWave ? 0u : at));
+    at = 0;
+    const uint64_t consumed = s_off + 2ull * base;
     if (inflight) {
       seg_land(ring, landed / kSegB, lane, seg);
       landed += kSegB;
       inflight = false;
     }
-    while (landed < e_off && landed < consumed + 4u * kWave + 2u) {
+    while (landed < e_off && landed < consumed + 2u * kWave + 2u) {
       seg_land(ring, landed / kSegB, lane, seg_block(A, landed / kSegB, lane, s_off, e_off));
       landed += kSegB;
     }
@@ -434,43 +342,312 @@ __device__ __forceinline__ void serial_chain_scalar(const GLB uint8_t* words, ui
       inflight = true;
     }
     wave_sync();
-    if (i0 == 0) {
-      w_lo = ring_word(lane);
-      w_hi = ring_word(kWave + lane);
-    } else if (pos - base >= (uint32_t)kWave) {           // one move keeps pos - base < 64
-      base += kWave;
-      w_lo = w_hi;
-      w_hi = ring_word(base + kWave + lane);
+    const uint32_t b = s_off + 2u * (base + lane);
+    win = (uint32_t)ring[b & (kRingB - 1u)] | ((uint32_t)ring[(b + 1u) & (kRingB - 1u)] << 8);
+    win = base + lane < n_words ? win : tail_word;
+  };
+  uint32_t acc = 0;            // lane j: the symbol index (lane * R + r) of step j of the batch
+  // One step: x becomes the next state, and lane j of acc takes the symbol's
+  // index. On the GPU the step is one asm block per R, in this order because
+  // issue is in order: a scalar instruction waits some 21 cycles for every
+  // vector instruction before it that writes a scalar register (compares,
+  // readlanes), whichever register it reads itself, so the compares come first,
+  // the arithmetic fills the wait, and the scalar instructions follow together.
+  // Wait states the hardware does not keep itself: two instructions between a
+  // vector write of a scalar register and a vector read of it (x: writelane and
+  // the next step's readlane of w; w, need, second: the arithmetic), one between
+  // a vector write and a readlane of it (y: s_addc).
+#ifdef BS_SIMT_CPU
+  // every lane finds the slot's symbol in the list by itself (an emulated
+  // ballot or readlane costs 64 fiber switches)
+  auto step = [&](uint32_t j) {
+    const uint32_t slot = x & ((1u << kLog) - 1u);
+    uint32_t lo = 0, hi = live;
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if ((syms[mid].x >> 16) <= slot) lo = mid; else hi = mid;
     }
-    // each step's output goes straight into lane j of acc (v_writelane): the
-    // LDS stage of serial_chain cost a v_mov and a ds_write per step, and its
-    // LDS count held up the wait for the next table load (a probe chain: 54.1
-    // against 50.4 ns per step)
-    const uint32_t cnt = min((uint32_t)kWave, n - i0);
-    if (cnt == (uint32_t)kWave) {
+    const uint32_t c = (syms[lo].x & 0xFFFFu) * (x >> kLog) + slot - (syms[lo].x >> 16);
+    if (c < kL) x = (c << 16) | (uint32_t)__builtin_amdgcn_readlane((int)win, (int)at++);
+    else x = c;
+    acc = lane == j ? lo : acc;
+  };
+#define BS_STEP(j) step(j)
+#else
+#define BS_STEP1(j)                                                                                              \
+  {                                                                                                                   \
+    uint32_t w, l, t, h, c, y;                                                                                        \
+    uint64_t need;                                                                                                    \
+    asm volatile("v_readlane_b32 %[w], %[win], %[at]\n\t"                                                             \
+                 "v_lshl_add_u32 %[t], %[x], %[top], %[first]\n\t"                                                    \
+                 "v_cmp_gt_u32 %[need], %[xb], %[x]\n\t"                                                              \
+                 "v_cmp_le_u32 vcc, %[t], %[last]\n\t"                                                                \
+                 "v_lshrrev_b32 %[h], %[log], %[x]\n\t"                                                               \
+                 "v_sub_u32 %[c], %[x], %[cf]\n\t"                                                                    \
+                 "v_mad_i32_i24 %[c], %[nf], %[h], %[c]\n\t"                                                          \
+                 "v_lshl_or_b32 %[y], %[c], 16, %[w]\n\t"                                                             \
+                 "v_cndmask_b32 %[y], %[c], %[y], %[need]\n\t"                                                        \
+                 "s_ff1_i32_b64 %[l], vcc\n\t"                                                                        \
+                 "s_bitcmp1_b64 %[need], %[l]\n\t"                                                                    \
+                 "s_addc_u32 %[at], %[at], 0\n\t"                                                                     \
+                 "v_readlane_b32 %[x], %[y], %[l]\n\t"                                                                \
+                 "v_writelane_b32 %[acc], %[l], %[step]"                                                              \
+                 : [x] "+s"(x), [at] "+s"(at), [acc] "+v"(acc), [w] "=&s"(w), [l] "=&s"(l), [t] "=&v"(t), [h] "=&v"(h), \
+                   [c] "=&v"(c), [y] "=&v"(y), [need] "=&s"(need)                                                     \
+                 : [cf] "v"(S.cf[0]), [nf] "v"(S.nf[0]), [xb] "v"(S.bound[0]), [first] "v"(S.first),                  \
+                   [last] "v"(S.last), [win] "v"(win), [log] "i"(kLog), [top] "i"(kTop), [step] "i"(j)                \
+                 : "vcc", "scc");                                                                                     \
+  }
+#define BS_STEP2(j)                                                                                              \
+  {                                                                                                                   \
+    uint32_t w, l, o, t, h, c, d, y;                                                                                  \
+    uint64_t need, second;                                                                                            \
+    asm volatile("v_readlane_b32 %[w], %[win], %[at]\n\t"                                                             \
+                 "v_lshl_add_u32 %[t], %[x], %[top], %[first]\n\t"                                                    \
+                 "v_lshrrev_b32 %[h], %[log], %[x]\n\t"                                                               \
+                 "v_cmp_ge_u32 %[second], %[t], %[begin]\n\t"                                                         \
+                 "v_cmp_le_u32 vcc, %[t], %[last]\n\t"                                                                \
+                 "v_sub_u32 %[c], %[x], %[cf]\n\t"                                                                    \
+                 "v_cndmask_b32 %[y], %[xb], %[xb1], %[second]\n\t"                                                   \
+                 "v_sub_u32 %[d], %[x], %[cf1]\n\t"                                                                   \
+                 "v_cmp_gt_u32 %[need], %[y], %[x]\n\t"                                                               \
+                 "v_mad_i32_i24 %[c], %[nf], %[h], %[c]\n\t"                                                          \
+                 "v_mad_i32_i24 %[d], %[nf1], %[h], %[d]\n\t"                                                         \
+                 "v_cndmask_b32 %[c], %[c], %[d], %[second]\n\t"                                                      \
+                 "v_lshl_or_b32 %[y], %[c], 16, %[w]\n\t"                                                             \
+                 "v_cndmask_b32 %[y], %[c], %[y], %[need]\n\t"                                                        \
+                 "s_ff1_i32_b64 %[l], vcc\n\t"                                                                        \
+                 "s_bitcmp1_b64 %[second], %[l]\n\t"                                                                  \
+                 "s_addc_u32 %[o], %[l], %[l]\n\t"                                                                    \
+                 "s_bitcmp1_b64 %[need], %[l]\n\t"                                                                    \
+                 "s_addc_u32 %[at], %[at], 0\n\t"                                                                     \
+                 "v_readlane_b32 %[x], %[y], %[l]\n\t"                                                                \
+                 "v_writelane_b32 %[acc], %[o], %[step]"                                                              \
+                 : [x] "+s"(x), [at] "+s"(at), [acc] "+v"(acc), [w] "=&s"(w), [l] "=&s"(l), [o] "=&s"(o),             \
+                   [t] "=&v"(t), [h] "=&v"(h), [c] "=&v"(c), [d] "=&v"(d), [y] "=&v"(y), [need] "=&s"(need),          \
+                   [second] "=&s"(second)                                                                             \
+                 : [cf] "v"(S.cf[0]), [cf1] "v"(S.cf[R - 1]), [nf] "v"(S.nf[0]), [nf1] "v"(S.nf[R - 1]),              \
+                   [xb] "v"(S.bound[0]), [xb1] "v"(S.bound[R - 1]), [first] "v"(S.first), [last] "v"(S.last),         \
+                   [begin] "v"(S.begin[R - 1]), [win] "v"(win), [log] "i"(kLog), [top] "i"(kTop), [step] "i"(j)       \
+                 : "vcc", "scc");                                                                                     \
+  }
+  auto step_many = [&](uint32_t j) {
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)win, (int)at), t = (x << kTop) + S.first;
+    const uint64_t hit = __ballot(t <= S.last);
+    uint32_t c = (uint32_t)__mul24(S.nf[0], (int)(x >> kLog)) + (x - S.cf[0]), sym = lane * R;
 #pragma unroll
-      for (uint32_t j = 0; j < (uint32_t)kWave; ++j) {
-        const uint32_t o = step();
-        BS_WRITELANE_I(acc, o, j);
-      }
-    } else {
-      for (uint32_t j = 0; j < cnt; ++j) {                 // the last, partial batch
-        const uint32_t o = step();
-        acc = lane == j ? o : acc;
-      }
+    for (int r = 1; r < R; ++r) {
+      const uint32_t cr = (uint32_t)__mul24(S.nf[r], (int)(x >> kLog)) + (x - S.cf[r]);
+      const bool ge = t >= S.begin[r];
+      c = ge ? cr : c;
+      sym = ge ? lane * R + r : sym;
     }
-    const uint32_t keep = acc & 0xFFu;
-    const uint32_t word = SE ? out_words[keep] : keep;
-    if (lane < cnt) {
+    const bool low = c < kL;
+    const uint64_t need = __ballot(low);
+    const uint32_t y = low ? (c << 16) | w : c, l = (uint32_t)__builtin_ctzll(hit);
+    x = (uint32_t)__builtin_amdgcn_readlane((int)y, (int)l);
+    at += (uint32_t)(need >> (l & 63u)) & 1u;
+    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)sym, (int)l);
+    // (a select on lane == j would hold the batch's 64 lane masks in registers)
+    asm volatile("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(acc) : "s"(o), "i"(j));
+  };
+#define BS_STEP(j)                       \
+  if constexpr (R == 1) BS_STEP1(j)      \
+  else if constexpr (R == 2) BS_STEP2(j) \
+  else step_many(j)
+#endif
+  auto settle = [&]() {
+    x = uni32(x);
+    at = uni32(at);
+    BS_SGPR_SETTLE(x, at);
+  };
+  // this lane's step of a batch at i0 out (cnt steps), its exponent into the tile's counts
+  auto emit = [&](uint32_t i0, uint32_t cnt) {
+    const uint32_t word = syms[min(acc, live - 1u)].y;
+    if (cnt == (uint32_t)kWave || lane < cnt) {
       if (SE) ((GLB uint16_t*)out)[(uint64_t)(i0 + lane) * stride] = (uint16_t)word;
-      else out[i0 + lane] = (uint8_t)keep;
+      else out[i0 + lane] = (uint8_t)word;
     }
     if (SE) tile_count(hist, ghist, word, lane, i0, cnt, n);
+  };
+  const uint32_t whole = n & ~(uint32_t)(kWave - 1);
+  for (uint32_t i0 = 0; i0 < whole; i0 += kWave) {
+#pragma unroll
+    for (uint32_t h0 = 0; h0 < kWave; h0 += kHalf) {
+      if (at >= kHalf) window();                         // uniform
+      settle();
+#pragma unroll
+      for (uint32_t j = 0; j < kHalf; ++j) {
+        BS_STEP(h0 + j);
+      }
+    }
+    emit(i0, kWave);
   }
+  if (whole < n) {                                       // the last, partial batch (a step's lane is a constant: 0)
+    uint32_t kept = 0;
+    for (uint32_t j = 0; j < n - whole; ++j) {
+      if (at >= kHalf) window();
+      settle();
+      BS_STEP(0);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)acc, 0);
+      kept = lane == j ? o : kept;
+    }
+    acc = kept;
+    emit(whole, n - whole);
+  }
+#undef BS_STEP
   if (SE) tile_count_end(ghist, lane, n, tps);
-  if (x != kL || pos != n_eff) {
+  if (at == kWave) at = 0;                               // an empty chain never opened its window
+  if (x != kL || base + at != n_eff) {
     if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
   }
+}
+
+// ---- mantissa chains, one per lane. The buckets of one exponent (one per stream of
+// a bf16_parallel_v1 tensor) share a decode table, so a wavefront decodes up to
+// 64 of them at once from one or two tables in LDS. A step costs more time than a
+// wave-wide chain's (an LDS read on the state's path), but it advances 64
+// chains, so the mantissas take a few wavefronts and leave the issue slots to the
+// SE chains, which set the launch's time. The host lists the buckets table by
+// table; a wavefront whose buckets have more than two tables takes two at a time.
+constexpr uint32_t kLaneRing = 32;                        // words in a lane's ring
+constexpr uint32_t kLaneTables = 2;                       // decode tables of a wavefront
+constexpr uint32_t kLaneB = kLaneTables * 4096 + kLaneRing * 2 * kWave;   // LDS bytes of a wavefront
+constexpr uint32_t kLaneSteps = 16;                       // steps between looks at the ring
+
+// Chains with at least this many buckets per table run one per lane: below it a
+// wavefront would hold buckets of three tables or more, and takes them in turns.
+constexpr uint32_t kLaneMin = 32;
+
+__device__ __forceinline__ void lane_chains(const bs_mant_bucket* __restrict__ buckets, uint32_t n_buckets,
+                                            uint32_t first, const uint32_t* __restrict__ tables, uint32_t n_tables,
+                                            uint64_t n_out, uint8_t* __restrict__ mant, LDS uint8_t* area,
+                                            int32_t* status) {
+  const uint32_t lane = __lane_id();
+  LDS uint32_t* tbl = (LDS uint32_t*)area;                // [table][slot]
+  LDS uint32_t* ring = (LDS uint32_t*)(area + kLaneTables * 4096);   // word p of a lane: half p & 1 of dword (p/2)*64 + lane
+  const bool have = first + lane < n_buckets;
+  const bs_mant_bucket B = buckets[have ? first + lane : first];
+  bool bad = have && (B.table >= n_tables || B.perm_begin + B.n > n_out);
+  if (bad) flag(status, BS_DEV_ERR_HEADER);
+  bool todo = have && !bad;
+  if (todo && B.x0 < kL) {
+    flag(status, BS_DEV_ERR_STREAM);
+    todo = false;
+  }
+  const GLB uint8_t* w = (const GLB uint8_t*)B.words;
+  const uint32_t n_eff = B.n_words + ((B.tail >> 16) & 1u), tail_word = B.tail & 0xFFFFu;
+  // words p .. p+7 (p a multiple of 8) as four dwords; past the stream its tail word
+  auto words8 = [&](uint32_t p) -> u32x4 {
+    u32x4 v;
+    if ((uint64_t)p + 8u <= B.n_words) {
+      typedef u32x4 __attribute__((aligned(1))) unaligned4;
+      v = *(const GLB unaligned4*)(w + 2ull * p);
+    } else {
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t a = p + 2 * k, b = a + 1;
+        v[k] = (a < B.n_words ? word_at(w, a) : tail_word) | (b < B.n_words ? word_at(w, b) : tail_word) << 16;
+      }
+    }
+    return v;
+  };
+  auto put8 = [&](uint32_t p, u32x4 v) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) ring[(((p >> 1) + k) & (kLaneRing / 2 - 1)) * kWave + lane] = v[k];
+  };
+  while (true) {
+    // the next tables still wanted, and whose lanes run now
+    uint64_t left = __ballot(todo);
+    if (left == 0) break;
+    bool run = false;
+    uint32_t slot0 = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kLaneTables; ++k) {
+      if (left == 0) break;                               // uniform
+      const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)B.table, (int)__builtin_ctzll(left));
+      const bool mine = todo && !run && B.table == t;
+      for (uint32_t i = lane; i < 1024; i += kWave) tbl[k * 1024 + i] = tables[(uint64_t)t * 1024u + i];
+      if (mine) {
+        run = true;
+        slot0 = k * 1024;
+      }
+      left &= ~__ballot(mine);
+    }
+    wave_sync();
+    todo = todo && !run;
+    if (run) {
+      uint32_t x = B.x0, pos = 0, ld = kLaneRing, r = 0;   // the ring holds words [pos, ld)
+      for (uint32_t p = 0; p < kLaneRing; p += 8) put8(p, words8(p));
+      GLB uint8_t* out = (GLB uint8_t*)(mant + B.perm_begin);
+      // the word at pos, read when pos moves: its latency passes under the next table read
+      auto next_word = [&]() {
+        return (uint32_t)((const LDS uint16_t*)ring)[2u * (((pos >> 1) & (kLaneRing / 2 - 1)) * kWave + lane) + (pos & 1u)];
+      };
+      uint32_t wnext = next_word();
+      auto step = [&]() -> uint32_t {
+        const uint32_t e = tbl[slot0 + (x & 1023u)];
+        const uint32_t c = __umul24(e & 0x7FFu, x >> 10) + ((e >> 11) & 0x3FFu);
+        const bool need = c < kL;
+        x = need ? (c << 16) | wnext : c;
+        pos += need ? 1u : 0u;
+        wnext = next_word();
+        return e >> 21;
+      };
+      for (; r + kLaneSteps <= B.n; r += kLaneSteps) {
+        while (ld - pos < kLaneSteps) {                   // rare: a block may take a word per step
+          put8(ld, words8(ld));
+          ld += 8;
+          wnext = next_word();
+        }
+        const uint32_t room = kLaneRing - (ld - pos);
+        u32x4 f0 = {0u, 0u, 0u, 0u}, f1 = {0u, 0u, 0u, 0u};
+        if (room >= 8) f0 = words8(ld);                   // in flight under the block, landed after it
+        if (room >= 16) f1 = words8(ld + 8);
+        u32x4 o;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+          uint32_t v = 0;
+#pragma unroll
+          for (uint32_t j = 0; j < 4; ++j) v |= (step() & 0x7Fu) << (8 * j);
+          o[k] = v;
+        }
+        if (room >= 8) put8(ld, f0);
+        if (room >= 16) put8(ld + 8, f1);
+        ld += room >= 16 ? 16u : room >= 8 ? 8u : 0u;
+        typedef u32x4 __attribute__((aligned(1))) unaligned4;
+        *(GLB unaligned4*)(out + r) = o;
+        wnext = next_word();                              // the word at pos may have landed only now
+      }
+      while (ld - pos < kLaneSteps) {
+        put8(ld, words8(ld));
+        ld += 8;
+      }
+      wnext = next_word();
+      for (; r < B.n; ++r) out[r] = (uint8_t)(step() & 0x7Fu);
+      if (x != kL || pos != n_eff) flag(status, BS_DEV_ERR_STREAM);
+    }
+    wave_sync();                                          // every lane is done with the tables
+  }
+}
+
+// List the live symbols of a decode table in LDS, in slot order: the slots
+// whose offset in their symbol is zero. `entry` gives slot i's {f | cf offset
+// (slot - cf), output}; one wavefront runs it. Returns their number (at most cap).
+template <uint32_t M, class Entry>
+__device__ __forceinline__ uint32_t list_symbols(LDS u32x2* syms, uint32_t cap, uint32_t lane, Entry entry) {
+  uint32_t live = 0;
+#pragma unroll 8
+  for (uint32_t i0 = 0; i0 < M; i0 += kWave) {
+    const uint32_t i = i0 + lane;
+    uint32_t f, off, out;
+    entry(i, f, off, out);
+    const bool starts = off == 0 && f != 0;
+    const uint64_t m = __ballot(starts);
+    const uint32_t r = live + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    if (starts && r < cap) syms[r] = u32x2{f | (i << 16), out};
+    live += (uint32_t)__popcll(m);
+  }
+  return min(live, cap);
 }
 
 // ---- tasks of a wave-serial launch. Every tensor of a batch is one task; its
@@ -523,20 +700,18 @@ __device__ __forceinline__ bs_ref_task pick_task(const bs_ref_task* __restrict__
 // xcd_slots(se_groups) workgroups serve the SE groups (task by
 // se_group_begin; their order is below): wave w of group j decodes SE stream
 // j*kSerWaves + w (element first + i*stride for symbol i) with the task's SE
-// table, built once per workgroup and shared.
+// symbols, listed once per workgroup and shared.
 // The rest are mantissa groups (task by mant_group_begin): wave w decodes
-// bucket j*kSerWaves + w into mant[perm_begin ...] with its own bucket table.
-// Sharing the 64 KB SE table lets a CU hold eight chains instead of two. The
-// host lists buckets longest first, so the four buckets of a group end at
+// bucket j*kSerWaves + w into mant[perm_begin ...], or, with kLaneMin buckets per
+// table or more, buckets 64 * (j*kSerWaves + w) .. + 63 (the groups past the
+// last such bucket exit at once).
+// The host lists buckets longest first, so the four buckets of a group end at
 // about the same time and the longest start first.
 //
 // The SE part of the grid has xcd_slots(se_groups) workgroups, a multiple of
 // kXcds: workgroup p serves SE group (p % kXcds) * (slots / kXcds) + p / kXcds
 // (none past the last group). Workgroups go to the XCDs round-robin, so each
-// XCD decodes one contiguous run of groups, which covers one or two tasks: the
-// scalar-cache form of an SE table (16 KB) then meets at most two tables in an
-// XCD's scalar caches, where seven interleaved tasks' tables missed often
-// enough to make each step ~40 % slower.
+// XCD decodes one contiguous run of groups, which covers one or two tasks.
 constexpr uint32_t kSerWaves = 4;
 constexpr uint32_t kXcds = 8;
 // A grid part of `count` workgroups dealt to the XCDs in contiguous blocks:
@@ -544,13 +719,13 @@ constexpr uint32_t kXcds = 8;
 __host__ __device__ constexpr uint64_t xcd_slots(uint32_t count) {
   return ((uint64_t)count + kXcds - 1) / kXcds * kXcds;
 }
-constexpr uint32_t kStageB = 128;      // per chain: 64 u16 outputs of a batch
+constexpr uint32_t kSeSyms = 512, kMantSyms = 128;
+constexpr uint32_t kSymB = kSeSyms * 8;   // one SE symbol list, or kSerWaves mantissa lists
+static_assert(kSerWaves * kMantSyms <= kSeSyms, "mantissa lists exceed the symbol area");
 constexpr uint32_t kHistB = 256 * 4;   // per SE chain: the exponent counts of its current tile
-// 78336: rings | SE table or kSerWaves mantissa tables | stages | tile counts.
-// Two groups fit the 160 KB of a CU (two of 81,920 B did not).
-constexpr uint32_t kSerLds = kSerWaves * kRingB + 4096 * 16 + kSerWaves * kStageB + kSerWaves * kHistB;
-static_assert(2 * kSerLds <= 160 * 1024 - 4096, "two chain groups per CU");
-static_assert(kSerWaves * 1024 * 16 <= 4096 * 16, "mantissa tables exceed the table area");
+// 48 KB: rings | symbols | tile counts (16 KB), or the lane-wise chains' tables and rings
+constexpr uint32_t kSerLds = kSerWaves * kLaneB;
+static_assert(kSerLds >= kSerWaves * kRingB + kSymB + kSerWaves * kHistB, "chain LDS");
 
 __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_task* __restrict__ tasks,
                                                                    uint32_t n_tasks, bs_ref_task single,
@@ -560,9 +735,8 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
   const uint32_t tid = threadIdx.x, lane = tid % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   LDS uint8_t* ring = (LDS uint8_t*)smem + wave * kRingB;
-  LDS u32x4* tbl_area = (LDS u32x4*)(smem + kSerWaves * kRingB);
-  LDS uint16_t* stage = (LDS uint16_t*)(smem + kSerWaves * kRingB + 4096 * 16 + wave * kStageB);
-  LDS uint32_t* hist = (LDS uint32_t*)(smem + kSerWaves * kRingB + 4096 * 16 + kSerWaves * kStageB + wave * kHistB);
+  LDS u32x2* syms = (LDS u32x2*)(smem + kSerWaves * kRingB);
+  LDS uint32_t* hist = (LDS uint32_t*)(smem + kSerWaves * kRingB + kSymB + wave * kHistB);
   const uint32_t slots = (uint32_t)xcd_slots(se_groups);  // the launch checked that it fits
   const bool se = blockIdx.x < slots;                     // uniform over the workgroup
   const uint32_t g = se ? (blockIdx.x % kXcds) * (slots / kXcds) + blockIdx.x / kXcds : blockIdx.x - slots;
@@ -572,7 +746,8 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
   const uint32_t begin = se ? T.se_group_begin : T.mant_group_begin;
   if (g < begin) return;
   const uint32_t local = g - begin, count = se ? T.n_streams : T.n_buckets;
-  if ((uint64_t)local * kSerWaves >= count) return;
+  const bool lanes = !se && T.n_buckets / kLaneMin >= T.n_tables;   // mantissa chains one per lane: 64 buckets a wave
+  if ((uint64_t)local * kSerWaves * (lanes ? kWave : 1u) >= count) return;
   if (!task_ok(T, work_bytes)) {
     if (local == 0 && tid == 0) flag(status, BS_DEV_ERR_HEADER);
     return;
@@ -580,35 +755,37 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
   const uint32_t c = local * kSerWaves + wave;            // this wave's stream or bucket (none when >= count)
   const uint64_t max_len = (uint64_t)serial_tiles(T.n_out, T.n_streams) * kTile;
   uint8_t* mant = work + T.work_offset;
-  const bool scalar_se = (T.flags & BS_REF_FLAG_SE_SCALAR) != 0;
   if (se) {
-    LDS uint32_t* out_words = (LDS uint32_t*)tbl_area;    // scalar-cache form: the 256 output words
-    if (scalar_se) {
-      for (uint32_t i = tid; i < 256; i += kSerWaves * kWave) out_words[i] = T.se_table[8192 + 4096 + i];
-    } else {
-      for (uint32_t i = tid; i < 4096; i += kSerWaves * kWave) {
-        const uint32_t lo = T.se_table[2 * i], sym = T.se_table[2 * i + 1];
-        const uint32_t word = (((sym >> 8) & 1u) << 15) | ((sym & 0xFFu) << 7);
-        tbl_area[i] = u32x4{lo & 0x1FFFu, lo >> 13, word, 0u};
-      }
-    }
+    // every wave lists the symbols alike (the same values to the same places)
+    const GLB u32x2* t = (const GLB u32x2*)T.se_table;
+    const uint32_t live = list_symbols<4096>(syms, kSeSyms, lane, [&](uint32_t i, uint32_t& f, uint32_t& off, uint32_t& o) {
+      const u32x2 e = t[i];
+      f = e.x & 0x1FFFu;
+      off = e.x >> 13;
+      o = (((e.y >> 8) & 1u) << 15) | ((e.y & 0xFFu) << 7);
+    });
     __syncthreads();
     if (c >= count) return;
     const bs_se_stream S = T.streams[c];
-    if (!stream_ok(S, max_len, T.n_out)) {
+    if (!stream_ok(S, max_len, T.n_out) || live == 0) {
       if (lane == 0) flag(status, BS_DEV_ERR_HEADER);
       return;
     }
+    __builtin_amdgcn_s_setprio(3);                        // the longest chains: issue before the mantissas'
     // the stream's tile counts: tps x 256 after the task's mantissa area
     const uint32_t tps = serial_tiles(T.n_out, T.n_streams);
     GLB uint32_t* ghist = (GLB uint32_t*)(work + T.work_offset + ((T.n_out + 255) & ~255ull)) + (uint64_t)c * tps * 256u;
-    if (scalar_se)
-      serial_chain_scalar<true>((const GLB uint8_t*)S.words, S.n_words, S.tail, S.x0, S.n,
-                                (const CST uint32_t*)(T.se_table + 8192), out_words, ring,
-                                (GLB uint8_t*)(T.out + S.first), S.stride, hist, ghist, tps, status);
-    else
-      serial_chain<true>((const GLB uint8_t*)S.words, S.n_words, S.tail, S.x0, S.n, tbl_area, ring, stage,
-                         (GLB uint8_t*)(T.out + S.first), S.stride, hist, ghist, tps, status);
+    auto run = [&](auto r) {
+      serial_chain<decltype(r)::value, true>((const GLB uint8_t*)S.words, S.n_words, S.tail, S.x0, S.n, syms, live, ring,
+                                             (GLB uint8_t*)(T.out + S.first), S.stride, hist, ghist, tps, status);
+    };
+    if (live <= 64) run(std::integral_constant<int, 1>{});
+    else if (live <= 128) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 8>{});
+  } else if (lanes) {
+    if ((uint64_t)c * kWave >= count) return;
+    lane_chains(T.buckets, T.n_buckets, c * kWave, T.mant_tables, T.n_tables, T.n_out, mant,
+                (LDS uint8_t*)smem + wave * kLaneB, status);
   } else {
     if (c >= count) return;
     const bs_mant_bucket B = T.buckets[c];
@@ -617,20 +794,20 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
       return;
     }
     const GLB uint32_t* t = (const GLB uint32_t*)T.mant_tables + (uint64_t)B.table * 1024u;
-    if (T.flags & BS_REF_FLAG_MANT_SCALAR) {
-      serial_chain_scalar<false>((const GLB uint8_t*)B.words, B.n_words, B.tail, B.x0, B.n, (const CST uint32_t*)t,
-                                 nullptr, ring, (GLB uint8_t*)(mant + B.perm_begin), 1u, nullptr, nullptr, 0u,
-                                 status);
+    syms += wave * kMantSyms;
+    const uint32_t live = list_symbols<1024>(syms, kMantSyms, lane, [&](uint32_t i, uint32_t& f, uint32_t& off, uint32_t& o) {
+      const uint32_t e = t[i];
+      f = e & 0x7FFu;
+      off = (e >> 11) & 0x3FFu;
+      o = (e >> 21) & 0x7Fu;
+    });
+    wave_sync();
+    if (live == 0) {
+      if (lane == 0) flag(status, BS_DEV_ERR_HEADER);
       return;
     }
-    LDS u32x4* tbl = tbl_area + wave * 1024u;
-    for (uint32_t i = lane; i < 1024; i += kWave) {
-      const uint32_t e = t[i];
-      tbl[i] = u32x4{e & 0x7FFu, (e >> 11) & 0x3FFu, (e >> 21) & 0x7Fu, 0u};
-    }
-    wave_sync();
-    serial_chain<false>((const GLB uint8_t*)B.words, B.n_words, B.tail, B.x0, B.n, tbl, ring, stage,
-                        (GLB uint8_t*)(mant + B.perm_begin), 1u, nullptr, nullptr, 0u, status);
+    serial_chain<2, false>((const GLB uint8_t*)B.words, B.n_words, B.tail, B.x0, B.n, syms, live, ring,
+                           (GLB uint8_t*)(mant + B.perm_begin), 1u, nullptr, nullptr, 0u, status);
   }
 }
 
@@ -725,13 +902,10 @@ __global__ __launch_bounds__(kWave) void place_kernel(const bs_ref_task* __restr
   if (__ballot(bad) != 0 && lane == 0) flag(status, BS_DEV_ERR_COUNT);
 }
 
-std::atomic<uint64_t> g_serial_lds{0};
-
 int launch_serial(const bs_ref_task* tasks, uint32_t n_tasks, const bs_ref_task& single, uint32_t se_groups,
                   uint32_t mant_groups, uint32_t tiles, uint32_t streams, uint8_t* work, uint64_t work_bytes,
                   int32_t* status, hipStream_t s) {
   if (xcd_slots(se_groups) + mant_groups > 0xFFFFFFFFull || xcd_slots(tiles) > 0xFFFFFFFFull) return BS_ERR_ARG;
-  bs_internal::ensure_lds_limit((const void*)serial_kernel, kSerLds, g_serial_lds);
   hipLaunchKernelGGL(serial_kernel, dim3((uint32_t)xcd_slots(se_groups) + mant_groups), dim3(kSerWaves * kWave),
                      kSerLds, s, tasks, n_tasks, single, se_groups, work, work_bytes, status);
   if (hipGetLastError() != hipSuccess) return BS_ERR_HIP;

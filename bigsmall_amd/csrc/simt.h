@@ -16,7 +16,7 @@
 #define BS_KEEP2(a, b) ((void)(a), (void)(b))
 #define BS_KEEP4(a, b, c, d) ((void)(a), (void)(b), (void)(c), (void)(d))
 #define BS_OPAQUE(x) ((void)(x))
-#define BS_WRITELANE_I(acc, v, j) ((acc) = __lane_id() == (uint32_t)(j) ? (uint32_t)(v) : (acc))
+#define BS_SGPR_SETTLE(a, b) ((void)(a), (void)(b))
 #define BS_LDS_ADD(p, v) ((void)atomicAdd((p), (v)))
 #define BS_BFE_U32(dst, x, off, width) ((dst) = ((uint32_t)(x) >> (off)) & ((1u << (width)) - 1u))
 #else
@@ -34,10 +34,10 @@
 #define BS_KEEP4(a, b, c, d) asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d))
 // Hides a value's provenance from the optimiser (it stays in a vector register).
 #define BS_OPAQUE(x) asm volatile("" : "+v"(x))
-// Lane j of the 32-bit register acc takes the wave-uniform value v (one
-// v_writelane_b32; v in a scalar register); j must be a constant once the
-// caller's loop is unrolled (a compile error otherwise).
-#define BS_WRITELANE_I(acc, v, j) asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(acc) : "s"(v), "i"(j))
+// Scalar registers a and b may be read by asm from here on: two wait states pass
+// since a vector instruction (readfirstlane) may have written them (the compiler
+// does not count them for asm).
+#define BS_SGPR_SETTLE(a, b) asm volatile("s_nop 1" : "+s"(a), "+s"(b))
 // dst = bits [off, off + width) of x in one v_bfe_u32 the optimiser cannot
 // rewrite (it turns a field extract followed by a scale into a shift and a
 // mask; kept whole, an LDS address from it is one v_lshl_add). off and width

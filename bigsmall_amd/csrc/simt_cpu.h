@@ -292,6 +292,9 @@ inline uint64_t __ballot(int pred) {
 inline int __any(int pred) { return __ballot(pred) != 0; }
 inline int __popcll(uint64_t v) { return __builtin_popcountll(v); }
 inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xFFFFFFu) * (b & 0xFFFFFFu); }
+inline int32_t __mul24(int32_t a, int32_t b) {      // the low 32 bits of the signed 24-bit product
+  return (int32_t)(uint32_t)((int64_t)((int32_t)((uint32_t)a << 8) >> 8) * (int64_t)((int32_t)((uint32_t)b << 8) >> 8));
+}
 inline int32_t atomicOr(int32_t* p, int32_t v) {
   const int32_t o = *p;
   *p = o | v;

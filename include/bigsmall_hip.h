@@ -262,10 +262,10 @@ uint32_t bs_refcodec_serial_tiles(uint64_t n_out, uint32_t n_streams);
  * previous one's end (the workgroups of a gap exit at once). The SE part of
  * the chain grid is dealt to the XCDs in bins: with total_se_groups rounded up
  * to 8C, slot p (which the round-robin dispatch sends to XCD p % 8) decodes SE
- * group (p % 8) * C + p / 8, so XCD j decodes groups [jC, (j+1)C). A caller
- * that places each task's SE groups inside one bin (gaps where needed) keeps
- * the tasks whose tables are read through the scalar cache on XCDs of their
- * own. */
+ * group (p % 8) * C + p / 8, so XCD j decodes groups [jC, (j+1)C); a caller
+ * may place each task's SE groups inside one bin (gaps where needed). A task
+ * with 32 buckets per table or more decodes 64 buckets per wavefront, fastest
+ * when they are listed table by table; any order decodes alike. */
 typedef struct {
     const bs_se_stream *streams;     /* n_streams SE stream descriptors */
     const uint32_t *se_table;        /* 4096 x {f | (slot-cf) << 13, symbol} u32 pairs */
@@ -284,14 +284,8 @@ typedef struct {
     uint32_t flags;                  /* BS_REF_FLAG_* */
 } bs_ref_task;
 
-/* bs_ref_task.flags. BS_REF_FLAG_SE_SCALAR: se_table continues after its 4096
- * pairs with the table's 4-byte form, 4096 u32 {index | f << 8 | (slot - cf)
- * << 20}, and 256 u32 output words (sign << 15 | exponent << 7 of the SE
- * symbol with that index), which a tensor with at most 256 live SE symbols,
- * none of frequency 4096, has; its SE chains then keep their state in scalar
- * registers and read that table through the scalar cache. BS_REF_FLAG_MANT_SCALAR:
- * the mantissa chains do the same with mant_tables. Either way the decoded
- * words are the same. */
+/* bs_ref_task.flags: accepted, without effect (they chose between two forms of
+ * the decode tables, which the chains no longer read). */
 #define BS_REF_FLAG_SE_SCALAR 1u
 #define BS_REF_FLAG_MANT_SCALAR 2u
 

@@ -243,3 +243,34 @@ def test_serial_batch_rejects_inconsistent_task(gpu):
         with pytest.raises(DecodeError):
             st.check("serial batch")
         assert outs[0].cpu().numpy().view(np.uint16).tobytes() == srcs[0].tobytes()
+
+
+@pytest.mark.parametrize("live", [1, 2, 63, 64, 65, 128, 129, 512])
+@pytest.mark.parametrize("codec", ["bf16_parallel_v1", "bf16_se_tans", "bf16_se_single_kernel"])
+def test_chain_symbol_counts(gpu, codec, live):
+    """Wave-serial chains hold 1, 2 or 8 sign/exponent symbols per lane: live symbol
+    counts on both sides of each line, one symbol of frequency 4096 among them, and
+    a last batch of fewer than 64 steps."""
+    rng = np.random.default_rng(live)
+    n = (1 << 16) + 37
+    se = np.sort(rng.permutation(512)[:live])
+    pick = np.concatenate([np.arange(live), np.minimum(rng.geometric(0.2, n - live) - 1, live - 1)])
+    w = ((se[rng.permutation(pick)] << 7) | rng.integers(0, 128, n)).astype(np.uint16)
+    _say(f"[ref] {codec} with {live} live symbols")
+    assert _decode(codec, CODECS[codec][0](w), n) == w.tobytes()
+
+
+@pytest.mark.parametrize("streams", [8, 31, 32, 33, 64, 100, 256])
+def test_lane_chain_stream_counts(gpu, streams):
+    """Mantissa buckets one per lane from 32 buckets per table on: stream counts on
+    both sides of that line, and counts for which a wavefront holds buckets of
+    several tables; bucket sizes that are no multiple of the step block, and
+    mantissas that take nearly a word per two steps and hardly any."""
+    rng = np.random.default_rng(streams)
+    n = (1 << 17) + 101
+    w = _bf16(rng.standard_normal(n) * 0.02)
+    flat = (w & 0xFF80 | np.minimum(rng.geometric(0.7, n), 127)).astype(np.uint16)
+    for name, words in (("gauss", w), ("skewed", flat)):
+        _say(f"[ref] bf16_parallel_v1, {streams} streams, {name}")
+        blob = oracle.par1_encode(words, streams)
+        assert _decode("bf16_parallel_v1", blob, n) == words.tobytes(), name
