@@ -30,7 +30,15 @@ import numpy as np
 from .. import _native
 
 M_SE, M_MANT = 4096, 1024
-SERIAL_MIN_ELEMENTS = 1 << 16   # from here on a wavefront per chain beats a lane per chain
+# From here on a wavefront per chain beats a lane per chain: at every size. MI355X, us per
+# launch, lane against wavefront: one element 29 / 20; bf16_parallel_v1 4,096 elements 65 / 26,
+# 65,535 371 / 46; bf16_se_tans 1,024 372 / 59, 65,535 21,891 / 2,244. The lane form keeps the
+# blobs whose streams are longer than the placement tiles cover (serial_ok).
+SERIAL_MIN_ELEMENTS = 1
+# A RefLaunch that is not given its output address beforehand: the wave-serial tables hold that
+# address, so a launch to another one builds and uploads them first. Below this size such a
+# launch keeps the lane form, whose launch uploads nothing.
+SERIAL_MIN_UNBOUND = 1 << 16
 LANE_CHAINS_MIN = 32            # buckets per mantissa table from which a wavefront decodes 64 of them (csrc/refcodec_decode.hip)
 SE_ALPHABET, MANT_ALPHABET = 512, 128
 
@@ -365,8 +373,7 @@ def _pack(arrays: list[np.ndarray]) -> tuple[np.ndarray, list[int]]:
 def serial_ok(plan: RefPlan) -> bool:
     """The wave-serial path applies: a tensor of SERIAL_MIN_ELEMENTS or more
     whose streams each hold at most ceil(n / streams) symbols (every blob the
-    reference's encoders write; a smaller tensor decodes as fast with one lane
-    per chain)."""
+    reference's encoders write)."""
     max_len = max((n for _, _, _, n in plan.se_streams), default=0)
     return plan.n >= SERIAL_MIN_ELEMENTS and len(plan.se_streams) > 0 and max_len <= -(-plan.n // len(plan.se_streams))
 
@@ -475,11 +482,11 @@ class RefBatch:
 
 class RefLaunch:
     """Device-side tables and descriptors of one parsed blob (kept alive until
-    the decode launched from them has completed). A tensor of
-    SERIAL_MIN_ELEMENTS or more decodes with one wavefront per chain (a
-    one-task bs_refcodec_decode_serial_batch, whose tables are built for one
-    output address: pass `out_ptr` here to build them before the first
-    launch); a smaller one with one lane per chain (bs_refcodec_decode)."""
+    the decode launched from them has completed). With `out_ptr`, or from
+    SERIAL_MIN_UNBOUND elements on, a tensor decodes with one wavefront per
+    chain (a one-task bs_refcodec_decode_serial_batch, whose tables are built
+    for one output address: pass it here to build them before the first
+    launch); else with one lane per chain (bs_refcodec_decode)."""
 
     def __init__(self, plan: RefPlan, blob_ptr: int, device, out_ptr: int | None = None):
         import torch
@@ -488,7 +495,7 @@ class RefLaunch:
         self.n = plan.n
         self.plan, self.blob_ptr, self.device = plan, blob_ptr, device
         self._batch = None
-        self.serial = serial_ok(plan)
+        self.serial = serial_ok(plan) and (out_ptr is not None or plan.n >= SERIAL_MIN_UNBOUND)
         if self.serial:
             if out_ptr is not None:
                 self._batch = (out_ptr, RefBatch([(plan, blob_ptr, out_ptr)], device))

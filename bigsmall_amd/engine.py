@@ -15,8 +15,8 @@ one launch per codec family):
          bf16_chunked_v1 / fp8_chunked_v1 entry of the group,
        - one bs_refcodec_decode_serial_batch launch for the group's
          reference-format entries (bf16_parallel_v1, bf16_se_tans,
-         bf16_se_single_kernel) of 65,536 elements or more, so all their
-         chains run side by side, and bs_refcodec_decode per smaller one,
+         bf16_se_single_kernel), so all their chains run side by side (and
+         bs_refcodec_decode for one whose streams that path does not take),
        - one bs_zstd_decode launch for the group's zstd frames (`zstd`,
          `zstd_xor_delta` and the index streams of `special` lowcard
          entries), then bs_lut_expand per lowcard entry,

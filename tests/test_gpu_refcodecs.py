@@ -274,3 +274,28 @@ def test_lane_chain_stream_counts(gpu, streams):
         _say(f"[ref] bf16_parallel_v1, {streams} streams, {name}")
         blob = oracle.par1_encode(words, streams)
         assert _decode("bf16_parallel_v1", blob, n) == words.tobytes(), name
+
+
+@pytest.mark.parametrize("codec", list(CODECS))
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 1000, 5000])
+def test_small_tensors_on_both_paths(gpu, codec, n):
+    """A small tensor decodes alike with one wavefront per chain (its output
+    address given beforehand) and with one lane per chain (not given)."""
+    from bigsmall_amd.codecs import _refstreams
+    from bigsmall_amd.device import StatusWord, upload_bytes
+    torch = gpu
+    dev = torch.device("cuda", 0)
+    w = _bf16(np.random.default_rng(n).standard_normal(n) * 0.02)
+    blob = CODECS[codec][0](w)
+    d_blob = upload_bytes(blob, dev)
+    plan = _refstreams.PARSERS[codec](blob, n)
+    for bound in (True, False):
+        out = torch.zeros(n, dtype=torch.int16, device=dev)
+        _say(f"[ref] {codec} n={n} output address {'given' if bound else 'not given'}")
+        launch = _refstreams.RefLaunch(plan, d_blob.data_ptr(), dev, out.data_ptr() if bound else None)
+        assert launch.serial is bound
+        st = StatusWord(dev)
+        launch.launch(out.data_ptr(), st.ptr, torch.cuda.current_stream(dev).cuda_stream)
+        torch.cuda.synchronize()
+        st.check(codec)
+        assert out.cpu().numpy().tobytes() == w.tobytes()
