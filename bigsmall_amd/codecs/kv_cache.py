@@ -40,21 +40,24 @@ def compress_kv_entry(keys, values) -> bytes:
     import torch
     if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
         raise ValueError("compress_kv_entry requires BF16 keys and values")
-    gpu_blobs = None
     if keys.is_cuda and values.is_cuda and keys.numel() and values.numel():
+        # only the blobs come back (the encoder's arena holds a worst case for
+        # each), through pinned memory
         arena, spans = bf16_chunked.encode_device([keys, values], steps=KV_STEPS, compact=False)
-        host = arena.cpu().numpy()
-        gpu_blobs = [host[o:o + n].tobytes() for o, n in spans]
-    out = bytearray(struct.pack("<B", VERSION_GPU))
-    for i, t in enumerate((keys, values)):
+        host = torch.empty(sum(n for _, n in spans), dtype=torch.uint8, pin_memory=True)
+        blobs, pos = [], 0
+        for o, n in spans:
+            host[pos:pos + n].copy_(arena[o:o + n], non_blocking=True)
+            blobs.append(memoryview(host.numpy()[pos:pos + n]))
+            pos += n
+        torch.cuda.current_stream(arena.device).synchronize()
+    else:
+        blobs = [encode_words(_tensor_words(t)[0]) for t in (keys, values)]
+    parts = [struct.pack("<B", VERSION_GPU)]
+    for t, blob in zip((keys, values), blobs):
         shape = list(t.shape)
-        blob = gpu_blobs[i] if gpu_blobs is not None else encode_words(_tensor_words(t)[0])
-        out += struct.pack("<B", len(shape))
-        for s in shape:
-            out += struct.pack("<i", int(s))
-        out += struct.pack("<I", len(blob))
-        out += blob
-    return bytes(out)
+        parts += [struct.pack(f"<B{len(shape)}iI", len(shape), *(int(s) for s in shape), len(blob)), blob]
+    return b"".join(parts)
 
 
 def parse_kv_entry(data: bytes) -> list[tuple[list[int], int, int, int]]:
@@ -90,29 +93,31 @@ def parse_kv_entry(data: bytes) -> list[tuple[list[int], int, int, int]]:
 def decompress_kv_entry(data: bytes, device: str = "cuda"):
     """Inverse of compress_kv_entry: (keys, values) as bf16 tensors on `device`."""
     import torch
-    from ..device import ChunkBatch, ChunkJob, StatusWord, require_gpu, upload_bytes
+    from ..device import TASK_DTYPE, chunk_tasks, decode_chunk_tasks, require_gpu
     parts = parse_kv_entry(data)
     dev = require_gpu(device if str(device) != "cpu" else None)
-    buf = np.zeros(sum(((b + 255) & ~255) for _, _, _, b in parts) + 256, np.uint8)
-    jobs, outs, pos = [], [], 0
+    # one pinned buffer and one copy: status word, task table (its own 256 bytes), K's and V's blobs
+    pos = 512
+    assert 256 + 2 * TASK_DTYPE.itemsize <= pos
+    total = pos + sum((b + 255) & ~255 for _, _, _, b in parts)
+    d = torch.empty(total, dtype=torch.uint8, device=dev)
+    buf = torch.empty(total, dtype=torch.uint8, pin_memory=True).numpy()
+    outs, rows = [], []
     for shape, n, off, blen in parts:
-        buf[pos:pos + blen] = np.frombuffer(data, np.uint8, blen, off)
-        outs.append((torch.empty(shape if all(s > 0 for s in shape) else [n], dtype=torch.bfloat16, device=dev),
-                     pos, blen, n))
-        pos += (blen + 255) & ~255
-    d = upload_bytes(buf, dev)
-    for o, p, blen, n in outs:
+        o = torch.empty(shape if all(s > 0 for s in shape) else [n], dtype=torch.bfloat16, device=dev)
+        outs.append(o)
         if blen:
-            inf = bf16_chunked.info(bytes(buf[p:p + 32]))
+            inf = bf16_chunked.info(bytes(data[off:off + 32]))
             if inf.n != n:
                 raise ValueError(f"KV entry: blob holds {inf.n} elements, shape needs {n}")
-            jobs.append(ChunkJob(d.data_ptr() + p, blen, o.data_ptr(), n, inf.n_chunks, inf.plane_mode))
-    st = StatusWord(dev)
-    if jobs:
-        ChunkBatch(jobs, dev).launch(st)
-    torch.cuda.synchronize(dev)
-    st.check("KV entry")
-    k, v = outs[0][0], outs[1][0]
+            buf[pos:pos + blen] = np.frombuffer(data, np.uint8, blen, off)
+            rows.append((d.data_ptr() + pos, blen, o.data_ptr(), n, inf.n_chunks, inf.plane_mode))
+        pos += (blen + 255) & ~255
+    if rows:
+        t = np.array(rows, np.int64)
+        tasks, groups = chunk_tasks(t[:, 0], t[:, 1], t[:, 2], t[:, 3], t[:, 4])
+        decode_chunk_tasks(buf, d, tasks, groups, int(t[:, 5].max()), torch.cuda.current_stream(dev), "KV entry")
+    k, v = outs
     if str(device) == "cpu":
         return k.cpu(), v.cpu()
     return k, v

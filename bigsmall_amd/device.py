@@ -122,6 +122,41 @@ def inspect_chunk_header(blob_head: bytes):
     return info
 
 
+def chunk_tasks(blob_ptr, blob_bytes, out_ptr, n, n_chunks) -> tuple[np.ndarray, int]:
+    """The bs_chunk_task array of one batched launch from arrays (or scalars)
+    of its fields, and the launch's workgroup count."""
+    count = len(np.atleast_1d(blob_ptr))
+    tasks = np.zeros(count, TASK_DTYPE)
+    tasks["blob"], tasks["blob_bytes"], tasks["out"] = blob_ptr, blob_bytes, out_ptr
+    tasks["n"], tasks["n_chunks"] = n, n_chunks
+    if np.any(tasks["blob"] % 16) or np.any(tasks["out"] % 16):
+        raise ValueError("BSCK blobs and their outputs must be 16-byte aligned on the device")
+    per = _native.lib().bs_chunk_chunks_per_group()
+    groups = (tasks["n_chunks"].astype(np.int64) + per - 1) // per
+    ends = np.cumsum(groups)
+    tasks["wg_begin"] = ends - groups
+    return tasks, int(ends[-1]) if count else 0
+
+
+def decode_chunk_tasks(buf: np.ndarray, d_buf, tasks: np.ndarray, groups: int, max_mode: int, stream, what: str) -> None:
+    """Decode `tasks` (chunk_tasks) and wait for it; raises DecodeError on a bad
+    status. buf is pinned host memory and d_buf a device buffer of its size:
+    the status word at 0, the task table at 256, and from there on whatever the
+    caller placed in it (blobs); one copy on `stream` (a torch stream) brings
+    all of it over, and one copy back brings the status."""
+    import torch
+    buf[:256] = 0
+    buf[256:256 + tasks.nbytes] = tasks.view(np.uint8)
+    with torch.cuda.stream(stream):
+        d_buf.copy_(torch.from_numpy(buf), non_blocking=True)
+        d_buf.record_stream(stream)
+        st = StatusWord(view=d_buf[:4].view(torch.int32))
+        rc = _native.lib().bs_chunk_decode_batch(d_buf.data_ptr() + 256, len(tasks), groups, max_mode, st.ptr,
+                                                 stream_ptr(stream))
+        _native.check(rc, "bs_chunk_decode_batch")
+        st.check(what)                    # a copy on `stream`: waits for the decode
+
+
 class ChunkBatch:
     """A prepared batched launch: a device array of bs_chunk_task and its grid
     size. Reusable: launch() may be called repeatedly (e.g. for timing)."""

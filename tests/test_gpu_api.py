@@ -575,3 +575,31 @@ def test_compress_reference_formats_round_trip(tmp_path, kw):
     out = decoder.load(p)
     for k, v in src.items():
         assert _bytes(out[k]) == _bytes(v), k
+
+
+@pytest.mark.parametrize("block_shape", [(2, 16, 8), (1, 5, 3)])
+def test_kv_block_requests_in_one_table(tmp_path, block_shape):
+    """Requests over several layers, repeated and empty id lists among them, on the
+    current stream and on another one while the cache is still being filled:
+    every block equals its source (blocks of a multiple of 8 elements, and
+    blocks whose outputs sit at a padded stride)."""
+    import torch
+    from bigsmall_amd.kv_cache_manager import CompressedKVCache
+    heads, tokens, dim = block_shape
+    cache = CompressedKVCache(device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    src = {}
+    side = torch.cuda.Stream()
+    requests = [(0, [3, 0, 3]), (1, []), (2, [1]), (0, [2])]
+    for layer in range(3):
+        k, v = (torch.randn(heads, 4 * tokens, dim, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+        cache.set_blocks(layer, k, v, block_tokens=tokens)
+        src[layer] = (k, v)
+    for stream in (None, side):
+        print(f"[kv] requests {requests} on {'another' if stream else 'the current'} stream", flush=True)
+        got = cache.get_blocks_multi(requests, stream=stream)
+        for (layer, ids), kv in zip(requests, got):
+            for out, whole in zip(kv, src[layer]):
+                assert out.shape == (len(ids), heads, tokens, dim) and out.is_contiguous()
+                for j, b in enumerate(ids):
+                    assert torch.equal(out[j].view(torch.int16), whole[:, b * tokens:(b + 1) * tokens].contiguous().view(torch.int16))
