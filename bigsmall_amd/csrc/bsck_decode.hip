@@ -852,12 +852,12 @@ __device__ __forceinline__ void progress_priority(uint32_t blk, uint32_t nblk, b
 
 // Decode one chunk with one wavefront: K interleaved states per lane, MODE =
 // plane mode, EB = element bytes (2 for pair mode, whose elements are byte
-// pairs), PARTIAL = chunk may be shorter than 64*K*steps (the tensor's last
+// pairs), nc elements (fewer than 64*K*steps only in the tensor's last
 // chunk), CODER = 0 rANS, 1 tANS. n_words is the chunk table's count: renorm
 // words (rANS) or stream bits (tANS, whose stream is whole u32 words). fl:
 // bit 0 = the later of its CU's two workgroups, bit 1 = tANS states at the
 // stream head (coder 2; the stream then holds at least their 12 * 64K bits).
-template <int K, int MODE, int EB, bool PARTIAL, int CODER>
+template <int K, int MODE, int EB, int CODER>
 __device__ __forceinline__ void decode_chunk(const LDS uint64_t* __restrict__ tbl, LDS uint16_t* wring,
                                              LDS uint8_t* pring, LDS uint8_t* stage,
                                              const GLB uint8_t* __restrict__ cbase, uint32_t n_words,
@@ -943,7 +943,12 @@ __device__ __forceinline__ void decode_chunk(const LDS uint64_t* __restrict__ tb
 
   LDS uint16_t* prog = (LDS uint16_t*)((LDS uint8_t*)tbl + (kProgOff - kTblOff));   // kWaves entries
   const uint32_t pwave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t blk = 0;;) {
+  // Whole pairs of blocks take the unmasked path: all of a full chunk, and all
+  // but the last pair of the tensor's partial chunk, whose elements are in
+  // order (a partial chunk that ran masked from its start took 86 us of a launch
+  // that is done in 66 without one). The rest, if any, runs masked below.
+  const uint32_t whole = (nc / (2u * G::kBlkElems)) * 2u;          // blocks
+  for (uint32_t blk = 0; blk < whole;) {
     {
       // publish this wave's pair count and take the workgroup's lowest (0xFFFF:
       // no chunk, or done); a stale entry is lower than the true one, so the
@@ -966,38 +971,44 @@ __device__ __forceinline__ void decode_chunk(const LDS uint64_t* __restrict__ tb
     land_segments<K, RM>(S, F, wring, pring, C.lane);
     refill<K, RM, MAXB>(S, F, C, wring, pring);
     wave_sync();
-    if (PARTIAL && blk > 0) flush_half<K, EB, PARTIAL, G::kBlock / 2>(2 * blk - 1, C, stage);
     request_segments<K, RM>(S, F, C);
     if (RM == 1) {
       F.pl[0] = load_plane<K>(C.dplane, C.pstride, min(blk + 2, C.nblk - 1), C.lane);
       F.pl[1] = load_plane<K>(C.dplane, C.pstride, min(blk + 3, C.nblk - 1), C.lane);
     }
     wave_sync();
-    decode_block<K, MODE, EB, PARTIAL, CODER>(blk, cur0, S, F, C, tbl, wring, pring, stage);
-    if (PARTIAL && blk + 1 >= C.nblk) break;
+    decode_block<K, MODE, EB, false, CODER>(blk, cur0, S, F, C, tbl, wring, pring, stage);
     // ---- second block of the pair
     refill<K, RM, MAXB>(S, F, C, wring, pring);
     wave_sync();
-    if (PARTIAL) flush_half<K, EB, PARTIAL, G::kBlock / 2>(2 * blk + 1, C, stage);
-    decode_block<K, MODE, EB, PARTIAL, CODER>(blk + 1, cur1, S, F, C, tbl, wring, pring, stage);
+    decode_block<K, MODE, EB, false, CODER>(blk + 1, cur1, S, F, C, tbl, wring, pring, stage);
     blk += 2;
     if (blk >= C.nblk) break;
-    if (!PARTIAL) {
-      // The pair's loads were followed by its output stores: vmcnt(stores)
-      // lands the loads and leaves the stores in flight. Stating it gives the
-      // compiler's wait-count tracking an exact state here; the uses below
-      // keep its own waits for these registers at this point.
-      __builtin_amdgcn_s_waitcnt(wait_vm(stores_per_pair<K, RM, EB, PARTIAL>()));
-      if (RM == 1) { consume_plane(F.pl[0]); consume_plane(F.pl[1]); }
-      BS_KEEP2(F.w[0].x, F.w[1].x);
-      if (RM == 2) BS_KEEP2(F.p[0].x, F.p[1].x);
-    }
+    // The pair's loads were followed by its output stores: vmcnt(stores)
+    // lands the loads and leaves the stores in flight. Stating it gives the
+    // compiler's wait-count tracking an exact state here; the uses below
+    // keep its own waits for these registers at this point.
+    __builtin_amdgcn_s_waitcnt(wait_vm(stores_per_pair<K, RM, EB, false>()));
+    if (RM == 1) { consume_plane(F.pl[0]); consume_plane(F.pl[1]); }
+    BS_KEEP2(F.w[0].x, F.w[1].x);
+    if (RM == 2) BS_KEEP2(F.p[0].x, F.p[1].x);
   }
-  // a partial chunk's last staged half: the second half of its last block, or
-  // the first if that block has at most half a block of steps
-  if (PARTIAL) {
+  if (whole < C.nblk) {                    // the partial chunk's last one or two blocks
+    land_segments<K, RM>(S, F, wring, pring, C.lane);
+    refill<K, RM, MAXB>(S, F, C, wring, pring);
     wave_sync();
-    flush_half<K, EB, PARTIAL, G::kBlock / 2>((C.nsteps - 1) / (G::kBlock / 2), C, stage);
+    request_segments<K, RM>(S, F, C);
+    decode_block<K, MODE, EB, true, CODER>(whole, F.pl[0], S, F, C, tbl, wring, pring, stage);
+    if (whole + 1 < C.nblk) {
+      refill<K, RM, MAXB>(S, F, C, wring, pring);
+      wave_sync();
+      flush_half<K, EB, true, G::kBlock / 2>(2 * whole + 1, C, stage);
+      decode_block<K, MODE, EB, true, CODER>(whole + 1, F.pl[1], S, F, C, tbl, wring, pring, stage);
+    }
+    // the last staged half: the second half of the last block, or the first if
+    // that block has at most half a block of steps
+    wave_sync();
+    flush_half<K, EB, true, G::kBlock / 2>((C.nsteps - 1) / (G::kBlock / 2), C, stage);
   }
   // segments requested but never landed need no wait: nothing reads them
   if (C.lane == 0) *(volatile LDS uint16_t*)(prog + pwave) = 0xFFFFu;   // out of the workgroup's lowest
@@ -1012,7 +1023,7 @@ __device__ __forceinline__ void decode_chunk(const LDS uint64_t* __restrict__ tb
   if (bad) report(status, BS_DEV_ERR_STREAM);
 }
 
-template <int K, int EB, bool PARTIAL, bool COMPACT, int CODER>
+template <int K, int EB, bool COMPACT, int CODER>
 __device__ __forceinline__ void decode_chunk_mode(uint32_t mode, const LDS uint64_t* tbl, LDS uint16_t* wring,
                                                   LDS uint8_t* pring, LDS uint8_t* stage, const GLB uint8_t* cbase,
                                                   uint32_t nw, uint32_t np, const GLB uint8_t* dplane,
@@ -1020,48 +1031,43 @@ __device__ __forceinline__ void decode_chunk_mode(uint32_t mode, const LDS uint6
                                                   uint32_t nc, uint32_t nsteps, int32_t* status, uint32_t fl) {
   if constexpr (EB == 1) {   // byte symbols (no plane); exponent pairs run as 2-byte elements
     if (mode == 3)
-      decode_chunk<K, 3, 2, PARTIAL, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+      decode_chunk<K, 3, 2, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
     else
-      decode_chunk<K, 0, EB, PARTIAL, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+      decode_chunk<K, 0, EB, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
   } else {
     if (mode == 0) {
-      decode_chunk<K, 0, EB, PARTIAL, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+      decode_chunk<K, 0, EB, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
     } else if (mode == 1) {
-      decode_chunk<K, 1, EB, PARTIAL, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+      decode_chunk<K, 1, EB, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
     } else {
       if constexpr (COMPACT)
-        decode_chunk<K, 2, EB, PARTIAL, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+        decode_chunk<K, 2, EB, CODER>(tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
     }
   }
 }
 
 template <int K, bool COMPACT, int CODER>
-__device__ __forceinline__ void decode_chunk_c(uint32_t eb, bool partial, uint32_t mode, const LDS uint64_t* tbl,
+__device__ __forceinline__ void decode_chunk_c(uint32_t eb, uint32_t mode, const LDS uint64_t* tbl,
                                                LDS uint16_t* wring, LDS uint8_t* pring, LDS uint8_t* stage,
                                                const GLB uint8_t* cbase, uint32_t nw, uint32_t np,
                                                const GLB uint8_t* dplane, uint64_t pstride, GLB uint8_t* out,
                                                uint64_t ubase, uint64_t ustride, uint32_t nc, uint32_t nsteps,
                                                int32_t* status, uint32_t fl) {
-  if (eb == 2) {
-    if (partial) decode_chunk_mode<K, 2, true, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
-    else decode_chunk_mode<K, 2, false, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
-  } else {
-    if (partial) decode_chunk_mode<K, 1, true, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
-    else decode_chunk_mode<K, 1, false, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
-  }
+  if (eb == 2) decode_chunk_mode<K, 2, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+  else decode_chunk_mode<K, 1, COMPACT, CODER>(mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
 }
 
 template <int K, bool COMPACT>
-__device__ __forceinline__ void decode_chunk_k(uint32_t eb, bool partial, uint32_t mode, uint32_t coder,
+__device__ __forceinline__ void decode_chunk_k(uint32_t eb, uint32_t mode, uint32_t coder,
                                                const LDS uint64_t* tbl, LDS uint16_t* wring, LDS uint8_t* pring,
                                                LDS uint8_t* stage, const GLB uint8_t* cbase, uint32_t nw, uint32_t np,
                                                const GLB uint8_t* dplane, uint64_t pstride, GLB uint8_t* out,
                                                uint64_t ubase, uint64_t ustride, uint32_t nc, uint32_t nsteps,
                                                int32_t* status, uint32_t fl) {
   if (coder == 0)
-    decode_chunk_c<K, COMPACT, 0>(eb, partial, mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+    decode_chunk_c<K, COMPACT, 0>(eb, mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
   else
-    decode_chunk_c<K, COMPACT, 1>(eb, partial, mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
+    decode_chunk_c<K, COMPACT, 1>(eb, mode, tbl, wring, pring, stage, cbase, nw, np, dplane, pstride, out, ubase, ustride, nc, nsteps, status, fl);
 }
 
 template <bool COMPACT>
@@ -1374,7 +1380,6 @@ __global__ __launch_bounds__(kThreads) void bsck_decode_kernel(const bs_chunk_ta
   LDS uint8_t* pring = s_wring + wave * kRingBytes + Geo<1, 2>::kPRingOff;   // rANS compact chunks only
   LDS uint8_t* stage = s_stage + wave * kStageMax;
   GLB uint8_t* out = (GLB uint8_t*)T.out;
-  const bool partial = !full;
   const GLB uint8_t* dplane = split ? b + preg + chunk * pblk : nullptr;   // nullptr: inline after the stream
   const uint64_t pstride = split ? nf * pblk : pblk;
   // version 3 interleaves the full chunks' 512-element units; version 2 (and
@@ -1385,13 +1390,13 @@ __global__ __launch_bounds__(kThreads) void bsck_decode_kernel(const bs_chunk_ta
   // bit 0: the later of its CU's two workgroups; bit 1: tANS states at the stream head
   const uint32_t fl = (blockIdx.x >= first_round ? 1u : 0u) | (coder == 2 ? 2u : 0u);
   if (lanes == 64)
-    decode_chunk_k<1, COMPACT>(eb, partial, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
+    decode_chunk_k<1, COMPACT>(eb, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
                                out, ubase, ustride, nc, nsteps, status, fl);
   else if (lanes == 128)
-    decode_chunk_k<2, COMPACT>(eb, partial, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
+    decode_chunk_k<2, COMPACT>(eb, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
                                out, ubase, ustride, nc, nsteps, status, fl);
   else
-    decode_chunk_k<4, COMPACT>(eb, partial, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
+    decode_chunk_k<4, COMPACT>(eb, mode, coder, s_tbl, wring, pring, stage, cbase, nw, np, dplane, pstride,
                                out, ubase, ustride, nc, nsteps, status, fl);
 }
 

@@ -243,6 +243,38 @@ def test_spread_launches(torch_gpu, groups, last):
             assert o.cpu().numpy().tobytes() == w.tobytes()
 
 
+@pytest.mark.parametrize("kind", ["dense", "compact", "exact", "pairs", "bytes"])
+@pytest.mark.parametrize("lanes", [64, 128, 256])
+@pytest.mark.parametrize("coder", [0, 2])
+def test_partial_chunk_tails(torch_gpu, kind, lanes, coder):
+    """The tensor's partial chunk runs unmasked up to its last whole pair of
+    blocks and masked from there: tails of no, one and three pairs (1,024 or 2,048
+    elements by geometry) plus or minus one element, and around a block's end,
+    alone and after two full chunks, for every plane mode and coder."""
+    from bigsmall_amd.codecs import bf16_chunked as bc
+    rng = np.random.default_rng(lanes + coder)
+    steps = 64
+    mode = {"dense": 1, "compact": 2, "exact": 0, "pairs": 3, "bytes": 0}[kind]
+    tails = sorted({p * m + d for p in (1024, 2048) for m in (0, 1, 3) for d in (-1, 0, 1, 255, 512, 513)})
+    tails = [t for t in tails if 0 < t < lanes * steps]
+    _say(f"[bsck] {len(tails)} tails, {kind}, {lanes} lanes, coder {coder}")
+    for full in (0, 2):
+        for tail in tails:
+            n = full * lanes * steps + tail
+            if kind == "exact":
+                w = _bf16(1 + rng.standard_normal(n) * 0.01)
+            elif kind == "bytes":
+                w = rng.integers(0, 90, n).astype(np.uint8)
+            elif kind == "pairs":
+                w = rng.integers(0, 256, 2 * n).astype(np.uint8) & 0xB7      # 64 exponent pairs at most
+            else:
+                w = _bf16(rng.standard_normal(n) * 0.02)
+                if kind == "compact":
+                    w[rng.permutation(n)[: n // 2]] = 0
+            blob = bc.encode_array(w, steps=steps, mode=mode, lanes=lanes, coder=coder)
+            assert bc.decode(blob, {}, w.size, elem_bytes=w.itemsize) == w.tobytes(), (full, tail)
+
+
 @pytest.mark.parametrize("mode", [1, 2])
 def test_single_byte_corruptions_decode_or_raise(torch_gpu, mode):
     """Every single-byte corruption of a blob (header, symbol table, chunk
