@@ -54,7 +54,7 @@ struct Plan {
   uint32_t freq[256];         // per symbol
   uint32_t cum[256];          // per symbol
   uint32_t rcp[256];          // per symbol: multiplier for x / freq (see div_constants)
-  uint32_t shf[256];          // per symbol: its two shifts (s1 | s2 << 8)
+  uint32_t shf[256];          // per symbol: its shift and increment (s | inc << 8)
   uint32_t nsym, ok, pad0, pad1;
 };
 constexpr uint64_t kPlanBytes = (sizeof(Plan) + 255) & ~uint64_t(255);
@@ -72,17 +72,32 @@ __device__ __forceinline__ uint64_t chunk_elem(uint64_t k, uint64_t j, uint64_t 
   return k < nf ? ((j / kUnit) * nf + k) * kUnit + j % kUnit : nf * per + j;
 }
 
-// Constants for x / f with a fixed divisor 1 <= f <= 4096 and any 32-bit x, without a divide
-// instruction: Granlund and Montgomery, "Division by Invariant Integers using
-// Multiplication" (PLDI 1994), Figure 4.1. With l = ceil(log2 f),
-//   m = floor(2^32 * (2^l - f) / f) + 1,  s1 = min(l, 1),  s2 = max(l - 1, 0),
-//   t = mulhi(m, x),  x / f = (t + ((x - t) >> s1)) >> s2.
-__device__ __forceinline__ void div_constants(uint32_t f, uint32_t& m, uint32_t& shf) {
-  const uint32_t l = f > 1 ? 32u - (uint32_t)__clz(f - 1) : 0u;
-  m = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - f)) / f + 1);
-  shf = (l ? 1u : 0u) | ((l ? l - 1 : 0u) << 8);
+// Constants for x / f with a fixed divisor 1 <= f <= 4096 and x < f * 2^20 (what a state is after
+// its renormalisation), in one multiply: x / f = mulhi(m, x + inc) >> s. With k = floor(log2 f)
+// one of the two roundings of 2^(32+k) / f is exact over 32 bits: the upper one when its error
+// m * f - 2^(32+k) is at most 2^k (Granlund and Montgomery, "Division by Invariant Integers using
+// Multiplication", PLDI 1994), else the lower one with x + 1 (Robison, "N-Bit Unsigned Division
+// Via N-Bit Multiply-Add", ARITH 2005). A power of two takes m = 2^31 and one shift less; f = 1,
+// m = 2^32 - 1 and x + 1. x + 1 does not wrap: f = 4096 has inc = 0.
+__host__ __device__ inline void div_constants(uint32_t f, uint32_t& m, uint32_t& s_inc) {
+  const uint32_t k = 31u - (uint32_t)__builtin_clz(f);
+  const uint64_t top = (uint64_t)1 << (32 + k);
+  if (f == 1) {
+    m = 0xFFFFFFFFu;
+    s_inc = 1u << 8;
+  } else if ((f & (f - 1)) == 0) {
+    m = 1u << 31;
+    s_inc = k - 1;
+  } else {
+    const uint64_t up = top / f + 1;
+    const bool down = up * f - top > ((uint64_t)1 << k);
+    m = (uint32_t)(down ? up - 1 : up);
+    s_inc = k | (down ? 1u << 8 : 0u);
+  }
 }
-__host__ __device__ inline uint64_t scratch_bytes(uint32_t steps) { return 4ull * kLanes + 2ull * kLanes * steps; }
+// Per chunk: the states, the renorm words (filled from the end), and a slot that
+// the lanes without a word write to.
+__host__ __device__ inline uint64_t scratch_bytes(uint32_t steps) { return 4ull * kLanes + 2ull * kLanes * steps + 16; }
 
 __device__ __forceinline__ void flag(int32_t* status, int32_t bits) { atomicOr(status, bits); }
 
@@ -337,8 +352,7 @@ __global__ __launch_bounds__(kWave) void enc_plan_kernel(const bs_encode_task* _
 template <bool FULL>
 __device__ __forceinline__ void encode_steps(const GLB uint32_t* src2, const GLB uint16_t* src1, const SegMap& sm,
                                              uint32_t lane, uint32_t nc, uint32_t nsteps, uint32_t k, uint32_t nf,
-                                             uint32_t per, const uint32_t* s_fc, const uint32_t* s_m,
-                                             GLB uint16_t* words, uint32_t& wpos, uint32_t (&x)[2], bool plane_here,
+                                             uint32_t per, const LDS u32x4* s_tab, GLB uint8_t* words, uint32_t& wpos, uint32_t (&x)[2], bool plane_here,
                                              GLB uint8_t* plane, uint64_t pstride) {
   // this lane's two words of step t, packed (first | second << 16); 0 past the
   // end. A step's 128 elements lie in one unit, so their words are contiguous.
@@ -351,6 +365,11 @@ __device__ __forceinline__ void encode_steps(const GLB uint32_t* src2, const GLB
     const uint32_t j0 = t * kLanes + 2 * lane;
     if (j0 + 1 < nc) return src2[(w0 >> 1) + lane];
     return j0 < nc ? (uint32_t)src1[w0 + 2 * lane] : 0u;
+  };
+  // {f * 2^20 - 1, m, 4096 - f | inc << 24, s | cum << 20} of the two words' symbols
+  auto entries = [&](uint32_t w2, u32x4 (&e)[2]) {
+    e[0] = s_tab[(w2 >> 7) & 0xFFu];
+    e[1] = s_tab[(w2 >> 23) & 0xFFu];
   };
   const uint32_t nblk = (nsteps + kBlock - 1) / kBlock;
   uint32_t cur[kBlock];
@@ -372,41 +391,42 @@ __device__ __forceinline__ void encode_steps(const GLB uint32_t* src2, const GLB
       }
       *(GLB u32x4*)(plane + (uint64_t)b * pstride) = u32x4{pw[0], pw[1], pw[2], pw[3]};
     }
+    // table entries of the block's last step; each step reads the next one's
+    // before its own arithmetic, which covers their latency
+    u32x4 e[2], en[2];
+    entries(cur[kBlock - 1], e);
 #pragma unroll
     for (int q = (int)kBlock - 1; q >= 0; --q) {
       const uint32_t t = b * kBlock + (uint32_t)q;
-      if (!FULL && t >= nsteps) continue;                      // uniform: the last block may be short
-      const uint32_t j0 = t * kLanes + 2 * lane;
-      const uint32_t wv[2] = {cur[q] & 0xFFFFu, cur[q] >> 16};
+      if (q > 0) entries(cur[q - 1], en);
+      if (FULL || t < nsteps) {                                // uniform: the last block may be short
+        const uint32_t j0 = t * kLanes + 2 * lane;
 #pragma unroll
-      for (int g = 1; g >= 0; --g) {
-        const bool active = FULL || j0 + g < nc;
-        const uint32_t ex = (wv[g] >> 7) & 0xFFu;
-        const uint32_t fc = s_fc[ex], f = (fc >> 5) & 0x1FFFu, cm = (fc >> 18) & 0xFFFu;
-        uint32_t xv = x[g];
-        // renormalise while x >= f * 2^20 (never for f = 4096): f * 2^20 is a
-        // multiple of 2^20, so the test is x >> 20 >= f, in 32 bits
-        const bool emit = active && (xv >> 20) >= f;
-        const uint64_t m = __ballot(emit);
-        // the emitting lanes' words, lane-descending from wpos - 1: a lane's slot
-        // is the new wpos plus the emitting lanes below it
-        wpos -= (uint32_t)__popcll(m);
-        if (emit) {
-          words[wpos + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
-              (uint16_t)(xv & 0xFFFFu);
-          xv >>= 16;
+        for (int g = 1; g >= 0; --g) {
+          const bool active = FULL || j0 + g < nc;
+          uint32_t xv = x[g];
+          // renormalise while x >= f * 2^20 (never for f = 4096)
+          const bool emit = active && xv > e[g].x;
+          const uint64_t m = __ballot(emit);
+          // the emitting lanes' words, lane-descending from wpos - 1: a lane's slot
+          // is the new wpos plus the emitting lanes below it. Every lane stores (the
+          // others into the slot after the words): a branch around the store kept
+          // the steps around it apart.
+          wpos -= (uint32_t)__popcll(m);
+          uint32_t at = 2u * (wpos + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)));
+          asm("" : "+v"(at));                                  // (or the select below becomes that branch)
+          *(GLB uint16_t*)(words + (emit ? at : 2u * per)) = (uint16_t)(xv & 0xFFFFu);
+          xv = emit ? xv >> 16 : xv;
+          // xv' = (q << 12) + xv mod f + cum = xv + cum + q * (4096 - f), q = xv / f:
+          // q < 2^20 and 4096 - f < 2^13, a 24-bit product
+          const uint32_t q2 = __umulhi(e[g].y, xv + (e[g].z >> 24)) >> (e[g].w & 31u);
+          const uint32_t xn = xv + (e[g].w >> 20) + __umul24(q2, e[g].z);
+          x[g] = active ? xn : xv;
         }
-        if (active) {
-          // q = xv / f (Granlund-Montgomery with div_constants' m, s1, s2; the
-          // second shift by fc, whose bits 0..4 are s2), then xv' = (q << 12) + xv mod f + cum
-          // = xv + cum + q * (4096 - f): q < 2^20 (xv < f * 2^20 after the
-          // renormalisation) and 4096 - f < 2^13, a 24-bit product
-          const uint32_t mh = __umulhi(s_m[ex], xv);
-          const uint32_t q2 = (mh + ((xv - mh) >> ((fc >> 30) & 1u))) >> fc;
-          xv = xv + cm + __umul24(q2, 4096u - f);
-        }
-        x[g] = xv;
       }
+      e[0] = en[0];
+      e[1] = en[1];
     }
 #pragma unroll
     for (uint32_t q = 0; q < kBlock; ++q) cur[q] = nxt[q];
@@ -414,13 +434,20 @@ __device__ __forceinline__ void encode_steps(const GLB uint32_t* src2, const GLB
 }
 
 // One wavefront per chunk: lane l owns states l (group 0) and 64 + l (group 1);
-// state (g, l) codes element t*128 + 2l + g at step t.
+// state (g, l) codes element t*128 + 2l + g at step t. A full launch (16
+// wavefronts per CU) is bound by vector issue, a small one by the step's chain:
+// 42 instructions a step, two of them quarter-rate multiplies. With the entries
+// read a step ahead in one LDS read each, one multiply per division and the
+// stores without a branch, MI355X: 4,096 chunks of 256 steps (a KV layer of 32,768
+// tokens) 96.6 -> 77 us, 64 chunks 68.8 -> 49 us.
 __global__ __launch_bounds__(kWave) void enc_chunk_kernel(const bs_encode_task* __restrict__ tasks, uint32_t n_tasks,
                                                           uint32_t steps, const uint8_t* __restrict__ plans,
                                                           ChunkRec* __restrict__ recs, uint8_t* __restrict__ scratch) {
-  // per exponent: {s2:5, f:13, cum:12, s1:1} of its symbol (s2 in bits 0..4, where a
-  // shift reads its amount), and the divisor's multiplier
-  __shared__ uint32_t s_fc[256], s_m[256];
+  // per exponent, of its symbol: {f * 2^20 - 1, multiplier, 4096 - f | inc << 24, shift | cum <<
+  // 20}, one LDS read (4096 - f in the low 24 bits and the shift in the low 5, where the product
+  // and the shift read them)
+  __shared__ __attribute__((aligned(16))) uint32_t s_raw[256 * 4];
+  LDS u32x4* s_tab = (LDS u32x4*)s_raw;
   const uint32_t lane = threadIdx.x, cg = blockIdx.x;
   const uint32_t ti = task_of(tasks, n_tasks, cg);
   const bs_encode_task T = tasks[ti];
@@ -428,9 +455,8 @@ __global__ __launch_bounds__(kWave) void enc_chunk_kernel(const bs_encode_task* 
   const Plan* P = (const Plan*)(plans + ti * kPlanBytes);
   if (!task_ok(T, per) || cg < T.chunk_begin || cg - T.chunk_begin >= T.n_chunks || !P->ok) return;
   for (uint32_t i = lane; i < 256; i += kWave) {
-    const uint32_t sym = P->sym_of_exp[i], shf = P->shf[sym];
-    s_fc[i] = (shf >> 8) | (P->freq[sym] << 5) | (P->cum[sym] << 18) | ((shf & 1u) << 30);
-    s_m[i] = P->rcp[sym];
+    const uint32_t sym = P->sym_of_exp[i], shf = P->shf[sym], f = P->freq[sym];
+    s_tab[i] = u32x4{(f << 20) - 1u, P->rcp[sym], (kM - f) | (shf >> 8) << 24, (shf & 31u) | P->cum[sym] << 20};
   }
   __syncthreads();
   const uint64_t k = cg - T.chunk_begin, nf = T.n / per;
@@ -451,16 +477,16 @@ __global__ __launch_bounds__(kWave) void enc_chunk_kernel(const bs_encode_task* 
   const GLB uint32_t* src2 = (const GLB uint32_t*)T.src;   // two words per lane-step (even elements)
   const GLB uint16_t* src1 = (const GLB uint16_t*)T.src;
   uint8_t* chunk = scratch + (uint64_t)cg * scratch_bytes(steps);
-  GLB uint16_t* words = (GLB uint16_t*)(chunk + 4u * kLanes);   // capacity per; filled from the end
+  GLB uint8_t* words = (GLB uint8_t*)(chunk + 4u * kLanes);     // capacity per; filled from the end
   uint32_t x[2] = {kL, kL};
   uint32_t wpos = (uint32_t)per;
   const SegMap sm = seg_map(T);
   if (k < nf)
-    encode_steps<true>(src2, src1, sm, lane, nc, nsteps, (uint32_t)k, (uint32_t)nf, (uint32_t)per, s_fc, s_m, words,
-                       wpos, x, plane_here, plane, pstride);
+    encode_steps<true>(src2, src1, sm, lane, nc, nsteps, (uint32_t)k, (uint32_t)nf, (uint32_t)per, s_tab, words, wpos,
+                       x, plane_here, plane, pstride);
   else
-    encode_steps<false>(src2, src1, sm, lane, nc, nsteps, (uint32_t)k, (uint32_t)nf, (uint32_t)per, s_fc, s_m,
-                        words, wpos, x, false, plane, pstride);
+    encode_steps<false>(src2, src1, sm, lane, nc, nsteps, (uint32_t)k, (uint32_t)nf, (uint32_t)per, s_tab, words,
+                        wpos, x, false, plane, pstride);
   GLB uint32_t* st = (GLB uint32_t*)chunk;
   st[lane] = x[0];
   st[kWave + lane] = x[1];

@@ -279,3 +279,23 @@ def test_segmented_rows_reject_bad_views():
     with pytest.raises(ValueError):                     # segment starts not 8 words apart in multiples
         bc.encode_device_rows([torch.zeros(4 * 3 * 1028, dtype=torch.bfloat16, device=dev)
                                .view(4, 3, 1028)[:, :, :512].permute(1, 0, 2)])
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_quantised_frequencies_of_every_kind(seed):
+    """The encoder divides by each symbol's frequency with constants of three kinds
+    (powers of two, rounded up, rounded down): skewed exponent distributions whose
+    frequencies run from 1 to nearly 4096, against the host encoder's bytes."""
+    import torch
+    from bigsmall_amd.codecs import bf16_chunked as bc
+    rng = np.random.default_rng(seed)
+    n_exp = [1, 2, 3, 12, 60, 256][seed]
+    p = rng.dirichlet(np.full(n_exp, [1, 0.02, 0.5, 0.3, 0.2, 1][seed]))
+    exps = rng.permutation(256)[:n_exp]
+    e = np.concatenate([exps, rng.choice(exps, 200_000 - n_exp, p=p)])
+    w = ((rng.integers(0, 2, e.size) << 15) | (e << 7) | rng.integers(0, 128, e.size)).astype(np.uint16)
+    _say(f"[enc] {n_exp} exponents, largest share {p.max():.4f}")
+    t = torch.from_numpy(w.view(np.int16).copy()).view(torch.bfloat16).cuda()
+    for steps in (16, 256):
+        arena, [(off, ln)] = bc.encode_device([t], steps=steps)
+        assert arena[off:off + ln].cpu().numpy().tobytes() == bc.encode_array(w, steps=steps, mode=bc.MODE_DENSE, lanes=128)
