@@ -342,3 +342,21 @@ def test_delta_roundtrip_against_safetensors_and_bs_base(tmp_path):
     want = (np.frombuffer(ft["layer.1.weight"].tobytes(), np.uint8) ^
             np.frombuffer(base["layer.1.weight"].tobytes(), np.uint8)).tobytes()
     assert _host_bytes(plain["layer.1.weight"]) == want
+
+
+@pytest.mark.parametrize("distinct,skew", [(2, 1.0), (16, 1.0), (40, 0.9), (256, 0.97), (24, 0.55)])
+def test_huffman_streams_of_every_length(distinct, skew):
+    """Literal sections whose streams end anywhere in a piece of the parallel Huffman decode (pieces of 32 to
+    512 bits, 16 or 64 a round): one and four streams, codes of one to eleven bits, one round and several."""
+    rng = np.random.default_rng(distinct)
+    p = skew ** np.arange(distinct)
+    p /= p.sum()
+    sizes = [64, 65, 255, 256, 257, 511, 513, 1000, 1023, 1024, 1025, 2047, 4095, 4096, 4097, 8191, 20_001, 65_537,
+             131_072, 140_003]
+    raws = [rng.choice(distinct, n, p=p).astype(np.uint8).tobytes() for n in sizes]
+    frames = [zstd_lib.compress(r, lv) for r in raws for lv in (-5, 1, 19)]
+    want = [r for r in raws for _ in range(3)]
+    _say(f"huffman streams: {distinct} values, skew {skew}, {len(frames)} frames")
+    outs, lens, st = _decode_batch(frames, [len(w) for w in want])
+    assert st == 0 and lens == [len(w) for w in want]
+    assert all(o == w for o, w in zip(outs, want))
