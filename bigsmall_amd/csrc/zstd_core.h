@@ -25,7 +25,7 @@ constexpr uint32_t kLLLog = 9, kMLLog = 9, kOFLog = 8, kWeightLog = 6;
 constexpr uint32_t kLLMax = 35, kMLMax = 52, kOFMax = 31;
 constexpr uint32_t kStageBytes = 24u << 10;    // compressed blocks up to this size are read from shared memory
 constexpr uint32_t kHufGroups = 64;            // pieces of a literal section's streams decoded side by side
-constexpr uint32_t kHufGroupBits = 512;        // stream bits of a piece at most
+constexpr uint32_t kHufQuarterMax = 128;       // stream bits of a quarter of a piece at most
 
 enum : int32_t {
   kOk = 0,
@@ -47,7 +47,7 @@ struct FseCell {
 struct BuildScratch {
   int16_t norm[64];
   uint16_t start[64];                 // FSE construction: cells of the symbols before this one
-  uint8_t weight[256];
+  alignas(16) uint8_t weight[256];
   alignas(16) uint8_t spread[1u << kLLLog];   // FSE construction: symbol of each cell
 };
 // Per piece of a Huffman stream and bit of its start that a code may begin at:
@@ -69,6 +69,7 @@ struct ZState {
     HufScratch h;
   };
   uint32_t entry[kHufGroups];         // per piece: its first code's bit in it | symbols before it << 4
+  uint16_t mark[kHufGroups][3];       // the same within a piece at its second, third and last quarter
   struct {
     uint32_t bits, off, count;        // a Huffman stream: its bits, first byte, symbols
     uint32_t at;                      // the same as `entry` for the pieces still to come
@@ -137,6 +138,16 @@ struct BackBits {
   __host__ __device__ int64_t bits() const { return (int64_t)lo * 8 + have; }
   __host__ __device__ void refill() {         // as many whole bytes as fit, loaded together
     if (have > 56 || lo == 0) return;
+    if (lo >= 8 && have >= 0) {
+      // one load; a byte of which only the top bits fit is read again by the next refill, the same bits
+      uint64_t v;
+      __builtin_memcpy(&v, p + lo - 8, 8);
+      acc |= v >> have;
+      const uint32_t k = (uint32_t)(64 - have) >> 3;
+      have += (int32_t)(8 * k);
+      lo -= k;
+      return;
+    }
     const uint32_t want = (uint32_t)(64 - have) >> 3;
     const uint32_t k = lo < want ? lo : want;
     uint64_t v = 0;
@@ -388,6 +399,16 @@ __host__ __device__ inline uint32_t read_weights(ZState& z, const uint8_t* q, ui
   return nw > 255 ? 0 : nw;
 }
 
+// Weights i .. i+15 (i a multiple of 16) as four words, zeros from nw on.
+__host__ __device__ inline void load_weights(const uint8_t* weight, uint32_t nw, uint32_t i, uint32_t (&w)[4]) {
+  __builtin_memcpy(w, __builtin_assume_aligned(weight + i, 16), 16);
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t left = nw > i + 4 * k ? nw - (i + 4 * k) : 0u;
+    if (left < 4) w[k] &= (1u << (8 * left)) - 1u;
+  }
+}
+
 // Builds z.huf from the tree description at q, whose size is inside the
 // section: the weights, the implied last weight, then codes assigned by weight
 // and symbol. Every lane calls it; it ends with a sync, except on an error.
@@ -414,11 +435,17 @@ __host__ __device__ inline int32_t build_huffman(const Team& tm, ZState& z, cons
     nw = z.val[0];
     if (!nw) return kErrTable;
   }
+  // read sixteen at a time (zeros after the last): a read at a time waits for each
   uint32_t total = 0, top = 0;
-  for (uint32_t i = 0; i < nw; ++i) {
-    const uint32_t w = weight[i];
-    total += w ? 1u << ((w - 1) & 31u) : 0u;
-    top = w > top ? w : top;
+  for (uint32_t i = 0; i < nw; i += 16) {
+    uint32_t w4[4];
+    load_weights(weight, nw, i, w4);
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k) {
+      const uint32_t w = (w4[k >> 2] >> (8 * (k & 3))) & 0xFFu;
+      total += (1u << (w & 31u)) >> 1;
+      top = w > top ? w : top;
+    }
   }
   if (top > kHufLogMax || total == 0) return kErrTable;
   const uint32_t log = highbit(total) + 1;
@@ -434,9 +461,14 @@ __host__ __device__ inline int32_t build_huffman(const Team& tm, ZState& z, cons
     const uint32_t w = s < nw ? weight[s] : last;
     if (!w) continue;
     uint32_t pos = s < nw && last < w ? 1u << (last - 1) : 0u;
-    for (uint32_t r = 0; r < nw; ++r) {
-      const uint32_t v = weight[r];
-      pos += v && (v < w || (v == w && r < s)) ? 1u << (v - 1) : 0u;
+    for (uint32_t r = 0; r < nw; r += 16) {
+      uint32_t w4[4];
+      load_weights(weight, nw, r, w4);
+#pragma unroll
+      for (uint32_t k = 0; k < 16; ++k) {
+        const uint32_t v = (w4[k >> 2] >> (8 * (k & 3))) & 0xFFu;
+        pos += v < w + (r + k < s) ? (1u << v) >> 1 : 0u;
+      }
     }
     const uint32_t e = s | ((log + 1 - w) << 8), run = 1u << (w - 1);
     if (run < 4) {
@@ -462,6 +494,73 @@ __host__ __device__ inline uint32_t bits32(const uint8_t* s, uint32_t n, int32_t
   return (uint32_t)(v >> (o & 7));
 }
 
+// Walks NJ chains of codes of a stream q[0, n) of T bits through windows of 32
+// bits from bit `at` to `to` (`at` plus a multiple of 32; the stream may end
+// before it). `win` holds the 64 bits from `at` on, p[j] the bit of chain j's
+// next code in them, c[j] its symbols so far.
+template <uint32_t NJ>
+__host__ __device__ __forceinline__ void huf_walk(const ZState& z, const uint8_t* q, uint32_t n, uint32_t T, uint32_t at,
+                                                  uint32_t to, uint32_t log, uint64_t& win, uint32_t (&p)[NJ],
+                                                  uint32_t (&c)[NJ]) {
+  const uint32_t mask = (1u << log) - 1, sh = 64 - log;
+  for (; at < to && at < T; at += 32) {
+    const uint32_t lim = T - at < 32 ? T - at : 32, next = bits32(q, n, (int32_t)(T - at) - 96);
+    if (NJ == 1) {
+      while (p[0] < lim) {
+        p[0] += z.huf[(uint32_t)(win >> (sh - p[0])) & mask] >> 8;
+        ++c[0];
+      }
+    } else {
+      for (;;) {
+        bool any = false;
+#pragma unroll
+        for (uint32_t j = 0; j < NJ; ++j) any = any || p[j] < lim;
+        if (!any) break;
+#pragma unroll
+        for (uint32_t j = 0; j < NJ; ++j) {
+          const uint32_t bits = z.huf[(uint32_t)(win >> (sh - p[j])) & mask] >> 8;
+          const bool on = p[j] < lim;
+          p[j] += on ? bits : 0u;
+          c[j] += on;
+        }
+      }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < NJ; ++j) p[j] -= lim;
+    win = (win << 32) | next;
+  }
+}
+
+// The 64 bits of stream q from bit `at` on.
+__host__ __device__ __forceinline__ uint64_t huf_window(const uint8_t* q, uint32_t n, uint32_t T, uint32_t at) {
+  return ((uint64_t)bits32(q, n, (int32_t)(T - at) - 32) << 32) | bits32(q, n, (int32_t)(T - at) - 64);
+}
+
+// Chains o, o + 4, .. of NJ of one piece (quarters of gq bits from bit p0): their
+// ends into hop[], their places at the piece's inner quarters into m[j][].
+template <uint32_t NJ>
+__host__ __device__ __forceinline__ void huf_piece(const ZState& z, const uint8_t* q, uint32_t n, uint32_t T, uint32_t p0,
+                                                   uint32_t gq, uint32_t o, uint16_t* hop, uint16_t (&m)[3][3]) {
+  const uint32_t log = z.huf_log;
+  uint32_t p[NJ], c[NJ];
+#pragma unroll
+  for (uint32_t j = 0; j < NJ; ++j) {
+    p[j] = o + 4 * j;
+    c[j] = 0;
+  }
+  uint64_t win = huf_window(q, n, T, p0);
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    huf_walk<NJ>(z, q, n, T, p0 + k * gq, p0 + (k + 1) * gq, log, win, p, c);
+#pragma unroll
+    for (uint32_t j = 0; j < NJ; ++j) {
+      const uint16_t v = (uint16_t)(p[j] | (c[j] << 4));
+      if (k < 3) m[j][k < 3 ? k : 0] = v;
+      else if (o + 4 * j < log) hop[o + 4 * j] = v;
+    }
+  }
+}
+
 // The Huffman streams z.hs[0, ns) of one literal section at `s` (their sizes
 // checked), stream i's symbols to out + i * seg. Every lane calls it after a
 // sync; returns whether every stream ends where it must, after a sync.
@@ -469,89 +568,89 @@ __host__ __device__ inline uint32_t bits32(const uint8_t* s, uint32_t n, int32_t
 // A code's place is known only once all codes before it are, so a stream is a
 // serial chain: one lane per stream took 60 % of a small frame's time. But a code
 // is at most 12 bits long, so a piece of a stream can be entered at one of at
-// most 12 bits. Each lane takes a piece (kHufGroups of them in all streams, up
-// to kHufGroupBits long) and walks it from every such bit, four at a time, which
-// are independent chains; then the true walk hops from piece to piece, one step
-// each; then each lane walks its piece once more from the true bit and writes
-// its symbols. Walking counts symbols of at least one bit, so a stream is right
-// exactly when the walk ends on its last bit with the expected count.
-// MI355X, 65 frames of 4,096 four-bit indices, tables built by all lanes too:
-// 220 -> 74 us.
+// most 12 bits. The streams are cut into kHufGroups pieces, and four lanes (of as
+// many wavefronts) walk a piece from every such bit, up to three chains a lane;
+// then the true walk hops from piece to piece, one step each; the lane that
+// walked the true chain tells where it was at the piece's quarters, and four
+// lanes walk a quarter each and write its symbols. Walking counts symbols of at
+// least one bit, so a stream is right exactly when the walk ends on its last bit
+// with the expected count. MI355X, 65 frames of 4,096 four-bit indices: 220 -> 74 us
+// with tables built by all lanes and one wavefront per frame, 44 to 50 us with four
+// and the literals in LDS.
 template <class Team>
 __host__ __device__ __forceinline__ bool huf_streams(const Team& tm, ZState& z, const uint8_t* s, uint32_t ns,
                                                      uint32_t seg, uint8_t* out) {
+  constexpr uint32_t kItems = 4 * kHufGroups, kPerLane = (kItems + Team::size - 1) / Team::size;
   const uint32_t log = z.huf_log, per = kHufGroups / ns;
-  const uint32_t mask = (1u << log) - 1;
   uint32_t most = 0;
   for (uint32_t i = 0; i < ns; ++i) most = z.hs[i].bits > most ? z.hs[i].bits : most;
   for (uint32_t base = 0; base < most;) {
-    // the pieces of this round: whole 32-bit windows
-    const uint32_t even = ((most - base + per - 1) / per + 31u) & ~31u;
-    const uint32_t gb = even < kHufGroupBits ? even : kHufGroupBits;
-    for (uint32_t g = tm.lane(); g < kHufGroups; g += Team::size) {
-      const uint32_t st = g / per, T = z.hs[st].bits, p0 = base + (g - st * per) * gb;
-      if (p0 >= T) continue;
-      const uint32_t end = p0 + gb < T ? p0 + gb : T, n = (T >> 3) + 1;
-      const uint8_t* q = s + z.hs[st].off;
-      const uint64_t first = ((uint64_t)bits32(q, n, (int32_t)(T - p0) - 32) << 32) | bits32(q, n, (int32_t)(T - p0) - 64);
-      for (uint32_t o = 0; o < log; o += 4) {
-        uint32_t p[4], c[4];
-        for (uint32_t i = 0; i < 4; ++i) {
-          p[i] = o + i;
-          c[i] = 0;
-        }
-        uint64_t win = first;           // 64 bits from bit `at` on; a code starts in its first 32
-        for (uint32_t at = p0; at < end; at += 32) {
-          const uint32_t lim = end - at < 32 ? end - at : 32, next = bits32(q, n, (int32_t)(T - at) - 96);
-          while (p[0] < lim || p[1] < lim || p[2] < lim || p[3] < lim) {
+    // the pieces of this round: four quarters of whole 32-bit windows
+    const uint32_t even = ((most - base + 4 * per - 1) / (4 * per) + 31u) & ~31u;
+    const uint32_t gq = even < kHufQuarterMax ? even : kHufQuarterMax;
+    uint16_t m[kPerLane][3][3];
 #pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-              const uint32_t e = z.huf[(uint32_t)(win >> (64 - log - p[i])) & mask];
-              const bool on = p[i] < lim;
-              p[i] += on ? e >> 8 : 0u;
-              c[i] += on;
-            }
-          }
-          for (uint32_t i = 0; i < 4; ++i) p[i] -= lim;
-          win = (win << 32) | next;
-        }
-        for (uint32_t i = 0; i < 4; ++i)
-          if (o + i < log) z.h.hop[g * kHufLogMax + o + i] = (uint16_t)(p[i] | (c[i] << 4));
-      }
+    for (uint32_t i = 0; i < kPerLane; ++i) {
+      const uint32_t it = i * Team::size + tm.lane(), g = it % kHufGroups, o = it / kHufGroups;
+      if (it >= kItems || o >= log) continue;
+      const uint32_t st = g / per, T = z.hs[st].bits, p0 = base + (g - st * per) * 4 * gq;
+      if (p0 >= T) continue;
+      const uint8_t* q = s + z.hs[st].off;
+      const uint32_t n = (T >> 3) + 1;
+      uint16_t* hop = z.h.hop + g * kHufLogMax;
+      if (log <= 4) huf_piece<1>(z, q, n, T, p0, gq, o, hop, m[i]);
+      else if (log <= 8) huf_piece<2>(z, q, n, T, p0, gq, o, hop, m[i]);
+      else huf_piece<3>(z, q, n, T, p0, gq, o, hop, m[i]);
     }
     tm.sync();
     for (uint32_t st = tm.lane(); st < ns; st += Team::size) {
+      const uint32_t bits = z.hs[st].bits;
       uint32_t at = z.hs[st].at;
-      for (uint32_t g = 0; g < per && base + g * gb < z.hs[st].bits; ++g) {
+      for (uint32_t g = 0; g < per && base + g * 4 * gq < bits; ++g) {
         z.entry[st * per + g] = at;
-        const uint32_t hop = z.h.hop[(st * per + g) * kHufLogMax + (at & 15u)];
-        at = (at & ~15u) + hop;         // the low fields: the new bit, and symbols added above it
+        // the low fields: the new bit, and symbols added above it
+        at = (at & ~15u) + z.h.hop[(st * per + g) * kHufLogMax + (at & 15u)];
       }
       z.hs[st].at = at;
     }
     tm.sync();
-    for (uint32_t g = tm.lane(); g < kHufGroups; g += Team::size) {
-      const uint32_t st = g / per, T = z.hs[st].bits, p0 = base + (g - st * per) * gb;
-      if (p0 >= T) continue;
-      const uint32_t end = p0 + gb < T ? p0 + gb : T, n = (T >> 3) + 1, count = z.hs[st].count;
+#pragma unroll
+    for (uint32_t i = 0; i < kPerLane; ++i) {
+      const uint32_t it = i * Team::size + tm.lane(), g = it % kHufGroups, o = it / kHufGroups;
+      if (it >= kItems || o >= log) continue;
+      const uint32_t st = g / per;
+      if (base + (g - st * per) * 4 * gq >= z.hs[st].bits) continue;
+      const uint32_t e = z.entry[g] & 15u;
+#pragma unroll
+      for (uint32_t j = 0; j < 3; ++j)
+        if (o + 4 * j == e)
+          for (uint32_t k = 0; k < 3; ++k) z.mark[g][k] = m[i][j][k];
+    }
+    tm.sync();
+    for (uint32_t it = tm.lane(); it < kItems; it += Team::size) {
+      const uint32_t g = it % kHufGroups, k = it / kHufGroups, st = g / per, T = z.hs[st].bits;
+      const uint32_t a = base + ((g - st * per) * 4 + k) * gq;
+      if (a >= T) continue;
+      const uint32_t n = (T >> 3) + 1, count = z.hs[st].count, mask = (1u << log) - 1, sh = 64 - log;
       const uint8_t* q = s + z.hs[st].off;
       uint8_t* d = out + (uint64_t)st * seg;
-      uint32_t p = z.entry[g] & 15u, k = z.entry[g] >> 4;
-      uint64_t win = ((uint64_t)bits32(q, n, (int32_t)(T - p0) - 32) << 32) | bits32(q, n, (int32_t)(T - p0) - 64);
-      for (uint32_t at = p0; at < end; at += 32) {
-        const uint32_t lim = end - at < 32 ? end - at : 32, next = bits32(q, n, (int32_t)(T - at) - 96);
+      const uint32_t e = z.entry[g], v = k ? z.mark[g][k - 1] : e & 15u;
+      uint32_t p = v & 15u, j = (e >> 4) + (v >> 4);
+      uint64_t win = huf_window(q, n, T, a);
+      for (uint32_t at = a; at < a + gq && at < T; at += 32) {
+        const uint32_t lim = T - at < 32 ? T - at : 32, next = bits32(q, n, (int32_t)(T - at) - 96);
         while (p < lim) {
-          const uint32_t e = z.huf[(uint32_t)(win >> (64 - log - p)) & mask];
-          if (k < count) d[k] = (uint8_t)e;
-          ++k;
-          p += e >> 8;
+          const uint32_t h = z.huf[(uint32_t)(win >> (sh - p)) & mask];
+          if (j < count) d[j] = (uint8_t)h;
+          ++j;
+          p += h >> 8;
         }
         p -= lim;
         win = (win << 32) | next;
       }
     }
     tm.sync();
-    base += per * gb;
+    base += per * 4 * gq;
   }
   bool ok = true;
   for (uint32_t i = 0; i < ns; ++i) ok = ok && z.hs[i].at == z.hs[i].count << 4;
@@ -613,22 +712,26 @@ __host__ __device__ inline void team_fill(const Team& tm, uint8_t* d, uint8_t v,
 }
 template <class Team>
 __host__ __device__ inline void team_copy(const Team& tm, uint8_t* d, const uint8_t* s, uint64_t n) {
-  // d and s do not overlap: eight bytes per lane in flight while that many are left
-  uint64_t i = tm.lane();
-  for (; i + 7 * Team::size < n; i += 8 * Team::size) {
-    uint8_t v[8];
+  // d and s do not overlap: four bytes per lane in flight (past the end, the last byte again)
+  for (uint64_t i = tm.lane(); i < n; i += 4 * Team::size) {
+    uint8_t v[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) v[k] = s[i + k * Team::size];
+    for (uint32_t k = 0; k < 4; ++k) {
+      const uint64_t j = i + k * Team::size;
+      v[k] = s[j < n ? j : n - 1];
+    }
 #pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) d[i + k * Team::size] = v[k];
+    for (uint32_t k = 0; k < 4; ++k)
+      if (i + k * Team::size < n) d[i + k * Team::size] = v[k];
   }
-  for (; i < n; i += Team::size) d[i] = s[i];
 }
 
-// One compressed block b[0, n) (RFC 8878 3.1.1.3). rep: repeat offsets.
+// One compressed block b[0, n) (RFC 8878 3.1.1.3). rep: repeat offsets. Literals
+// that are not read in place go to near[0, room) if they fit, else to lit_far.
 template <class Team>
 __host__ __device__ __forceinline__ int32_t zstd_block(const Team& tm, ZState& z, const uint8_t* b, uint64_t n,
-                                                       Out& o, Rep& rep, uint8_t* lit_buf) {
+                                                       Out& o, Rep& rep, uint8_t* near, uint32_t room,
+                                                       uint8_t* lit_far) {
   if (n < 1) return kErrTruncated;
   const uint32_t ltype = b[0] & 3u, sf = (b[0] >> 2) & 3u;
   uint32_t lh, lsize, lcsize = 0;
@@ -656,6 +759,7 @@ __host__ __device__ __forceinline__ int32_t zstd_block(const Team& tm, ZState& z
   }
   if (lsize > kBlockMax) return kErrFormat;
   uint64_t pos = lh;
+  uint8_t* lit_buf = lsize <= room ? near : lit_far;
   const uint8_t* lit = lit_buf;
   if (ltype == 0) {                     // raw literals: read in place
     if (pos + lsize > n) return kErrTruncated;
@@ -885,9 +989,9 @@ __host__ __device__ int32_t zstd_frames(const Team& tm, ZState& z, const uint8_t
         if (bsize <= kStageBytes) {     // bit reads then come from shared memory, not global memory
           team_copy(tm, z.stage, src + ip, bsize);
           tm.sync();
-          e = zstd_block(tm, z, z.stage, bsize, o, rep, lit_buf);
+          e = zstd_block(tm, z, z.stage, bsize, o, rep, z.stage + bsize, kStageBytes - bsize, lit_buf);
         } else {
-          e = zstd_block(tm, z, src + ip, bsize, o, rep, lit_buf);
+          e = zstd_block(tm, z, src + ip, bsize, o, rep, z.stage, kStageBytes, lit_buf);
         }
         if (e) return e;
         ip += bsize;

@@ -9,11 +9,11 @@
 //                           (bigsmall/decoder.py:88-90, 190-198); with a base
 //                           given, the kernel XORs it into the output.
 //
-// One 64-lane workgroup per task decodes all frames of its input with the
+// One 256-lane workgroup per task decodes all frames of its input with the
 // team-parallel decoder of zstd_core.h: tables and the current compressed
 // block (when it is at most 24 KB) in LDS, under 40 KB in all; literals
-// of the current block in a 128 KiB slice of the work buffer, matches copied
-// by all lanes. Zstandard is a sequential format (each match may copy bytes
+// of the current block in LDS too where they fit beside it, else in a 128 KiB
+// slice of the work buffer, matches copied by all lanes. Zstandard is a sequential format (each match may copy bytes
 // of the one before), so a frame is not split across workgroups; the
 // reference's zstd entries are small (norm-weight indices, integer buffers)
 // and many of them go in one launch.
@@ -44,7 +44,7 @@ static __device__ __align__(256) uint8_t scratch[(uint64_t)BS_ZSTD_STATIC_MAX_TA
 namespace {
 
 struct DevTeam {
-  static constexpr uint32_t size = 64;
+  static constexpr uint32_t size = 256;
   __device__ uint32_t lane() const { return threadIdx.x; }
   __device__ void sync() const { __syncthreads(); }
 };
@@ -59,7 +59,9 @@ __device__ int32_t status_bits(int32_t e) {
   }
 }
 
-__global__ __launch_bounds__(64) void zstd_kernel(const bs_zstd_task* __restrict__ tasks, uint8_t* __restrict__ work,
+// Three workgroups per CU: left alone the compiler takes 232 vector registers, which
+// lets in two, at the same speed; 128 registers for four cost the two-chain walks 15 %.
+__global__ __launch_bounds__(256, 3) void zstd_kernel(const bs_zstd_task* __restrict__ tasks, uint8_t* __restrict__ work,
                                                   uint64_t* __restrict__ out_len, int32_t* __restrict__ status) {
   __shared__ bs_zstd::ZState z;
   const bs_zstd_task T = tasks[blockIdx.x];
@@ -71,7 +73,7 @@ __global__ __launch_bounds__(64) void zstd_kernel(const bs_zstd_task* __restrict
     if (e == bs_zstd::kOk && got != T.dst_len) e = bs_zstd::kErrOutput;
   }
   if (e == bs_zstd::kOk && T.xor_src) {        // a delta: dst ^= base (the frames are all written)
-    for (uint64_t i = threadIdx.x; i < T.dst_len; i += 64) T.dst[i] ^= T.xor_src[i];
+    for (uint64_t i = threadIdx.x; i < T.dst_len; i += DevTeam::size) T.dst[i] ^= T.xor_src[i];
   }
   if (threadIdx.x == 0) {
     out_len[blockIdx.x] = e ? 0 : got;
@@ -133,7 +135,7 @@ int bs_zstd_decode(const bs_zstd_task* d_tasks, uint32_t n_tasks, void* d_work, 
   if (!d_status || (n_tasks && (!d_tasks || !d_work || !d_out_len)) || n_tasks > 0x7FFFFFFFu) return BS_ERR_ARG;
   if (n_tasks == 0) return BS_OK;
   if (work_bytes < bs_zstd_work_bytes(n_tasks)) return BS_ERR_ARG;
-  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(64), 0, (hipStream_t)stream, d_tasks, (uint8_t*)d_work,
+  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(DevTeam::size), 0, (hipStream_t)stream, d_tasks, (uint8_t*)d_work,
                      d_out_len, d_status);
   return hipGetLastError() == hipSuccess ? BS_OK : BS_ERR_HIP;
 }
@@ -157,7 +159,7 @@ int bs_zstd_decode_static(const bs_zstd_task* d_tasks, uint32_t n_tasks, uint64_
   // the previous call's launch (on any stream) has finished with the array;
   // an event never recorded is complete
   if (order && hipStreamWaitEvent(s, g_scratch_done[dev], 0) != hipSuccess) return BS_ERR_HIP;
-  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(64), 0, s, d_tasks, (uint8_t*)g_scratch_ptr[dev], d_out_len,
+  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(DevTeam::size), 0, s, d_tasks, (uint8_t*)g_scratch_ptr[dev], d_out_len,
                      d_status);
   if (hipGetLastError() != hipSuccess) return BS_ERR_HIP;
   if (order && hipEventRecord(g_scratch_done[dev], s) != hipSuccess) return BS_ERR_HIP;
