@@ -203,18 +203,21 @@ __global__ __launch_bounds__(256) void enc_hist_kernel(const bs_encode_task* __r
   if (sum) atomicAdd(&((Plan*)(plans + ti * kPlanBytes))->hist[tid], sum);
 }
 
-// is candidate (c1, d1, i1) better than (c0, d0, i0)? up: larger c/d; down: smaller c/d; ties: lower index.
-// c < 2^32 (elements of one tensor) and d <= 8193, so the products fit in 64 bits.
-__device__ __forceinline__ bool better(bool up, uint64_t c1, uint64_t d1, uint32_t i1, uint64_t c0, uint64_t d0,
-                                       uint32_t i0) {
-  const uint64_t a = c1 * d0, b = c0 * d1;
-  if (a != b) return up ? a > b : a < b;
-  return i1 < i0;
-}
-
 __device__ __forceinline__ uint64_t shfl64(uint64_t v, uint32_t src_lane) {
   const uint32_t lo = __shfl((uint32_t)v, src_lane), hi = __shfl((uint32_t)(v >> 32), src_lane);
   return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+
+// The largest of the wavefront's 64 values, in every lane: DPP moves within the 16-lane rows and
+// then from row to row, to lane 63.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));   // row_shr:1
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));   // row_shr:2
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));   // row_shr:4
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));   // row_shr:8
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));   // row_bcast:15
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));   // row_bcast:31
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)kWave - 1);
 }
 
 // One wavefront per task. Lane l holds exponents 4l .. 4l+3, so symbol indices
@@ -267,26 +270,40 @@ __global__ __launch_bounds__(kWave) void enc_plan_kernel(const bs_encode_task* _
     sum += f[r];
   }
   for (uint32_t d = 1; d < kWave; d <<= 1) sum += (int64_t)shfl64((uint64_t)sum, lane ^ d);
-  // greedy corrections, one symbol per iteration (the same sequence as bsck_encode.cpp)
-  while (sum != (int64_t)kM) {
-    const bool up = sum < (int64_t)kM;
-    uint64_t bc = 0, bd = 1;
-    uint32_t bi = 0xFFFFFFFFu;
+  // Greedy corrections, one symbol per iteration (the same sequence as bsck_encode.cpp): up, the
+  // symbol of the largest c / (2f + 1); down, of the smallest c / (2f - 1) among those with f > 1;
+  // ties to the lower symbol. Two such quotients that differ do so by one part in c * d < 2^46 or
+  // more (c < 2^32, d <= 8193), so their doubles differ too and order as they do, and equal ones
+  // round alike. Their bits, complemented on the way down, are a key whose largest wins, 0 for no
+  // candidate; only the winner's changes. The wavefront's largest comes from two 32-bit maxima
+  // over DPP moves, the high halves' and then the low halves' of the lanes that have it.
+  // MI355X, 256 blocks of K and V: 9.8 us against 20.5 with cross products over shuffles.
+  const bool up = sum < (int64_t)kM;
+  auto key_of = [&](int r) -> uint64_t {
+    if (!c[r] || (!up && f[r] <= 1)) return 0;
+    const uint64_t k = __builtin_bit_cast(uint64_t, (double)(uint32_t)c[r] / (double)(int32_t)(up ? 2 * f[r] + 1 : 2 * f[r] - 1));
+    return up ? k : ~k;
+  };
+  uint64_t key[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (!c[r] || (!up && f[r] <= 1)) continue;
-      const uint64_t d = up ? 2 * f[r] + 1 : 2 * f[r] - 1;
-      if (bi == 0xFFFFFFFFu || better(up, c[r], d, sidx[r], bc, bd, bi)) { bc = c[r]; bd = d; bi = sidx[r]; }
-    }
-    for (uint32_t d = 1; d < kWave; d <<= 1) {
-      const uint64_t oc = shfl64(bc, lane ^ d), od = shfl64(bd, lane ^ d);
-      const uint32_t oi = __shfl(bi, lane ^ d);
-      if (oi != 0xFFFFFFFFu && (bi == 0xFFFFFFFFu || better(up, oc, od, oi, bc, bd, bi))) { bc = oc; bd = od; bi = oi; }
-    }
+  for (int r = 0; r < 4; ++r) key[r] = key_of(r);
+  for (int64_t left = up ? (int64_t)kM - sum : sum - (int64_t)kM; left > 0; --left) {
+    int br = 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (c[r] && sidx[r] == bi) f[r] += up ? 1 : -1;
-    sum += up ? 1 : -1;
+    for (int r = 1; r < 4; ++r) br = key[r] > (br == 0 ? key[0] : br == 1 ? key[1] : key[2]) ? r : br;
+    const uint64_t best = br == 0 ? key[0] : br == 1 ? key[1] : br == 2 ? key[2] : key[3];
+    const uint32_t hi = (uint32_t)(best >> 32), top = wave_max(hi);
+    const uint32_t lo = hi == top ? (uint32_t)best : 0u;
+    const uint32_t low = wave_max(lo);                   // by every lane, so not inside the test below
+    const uint64_t at = __ballot(hi == top && lo == low);
+    if (lane == (uint32_t)__builtin_ctzll(at)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r == br) {
+          f[r] += up ? 1 : -1;
+          key[r] = key_of(r);
+        }
+    }
   }
   // cumulative frequencies in symbol order
   int64_t fl = 0;

@@ -299,3 +299,19 @@ def test_quantised_frequencies_of_every_kind(seed):
     for steps in (16, 256):
         arena, [(off, ln)] = bc.encode_device([t], steps=steps)
         assert arena[off:off + ln].cpu().numpy().tobytes() == bc.encode_array(w, steps=steps, mode=bc.MODE_DENSE, lanes=128)
+
+
+@pytest.mark.parametrize("counts", [[5] * 3, [5] * 7, [3] * 100, [9] * 255, [1] * 200 + [400_000], [1, 2, 3] * 60,
+                                    [1] * 255 + [4096], [100_000, 99_999, 100_001, 1]])
+def test_quantiser_corrections_and_ties(counts):
+    """The frequencies' corrections to a sum of 4096, up and down: symbols that tie (the lower
+    one wins), symbols already at 1 (never lowered), quotients that differ in their last place."""
+    import torch
+    from bigsmall_amd.codecs import bf16_chunked as bc
+    e = np.repeat(np.arange(len(counts)), counts)
+    e = np.random.default_rng(len(counts)).permutation(e)
+    w = (e << 7).astype(np.uint16)
+    _say(f"[enc] {len(counts)} exponents, {e.size} elements")
+    t = torch.from_numpy(w.view(np.int16).copy()).view(torch.bfloat16).cuda()
+    arena, [(off, ln)] = bc.encode_device([t], steps=16)
+    assert arena[off:off + ln].cpu().numpy().tobytes() == bc.encode_array(w, steps=16, mode=bc.MODE_DENSE, lanes=128)
