@@ -1,5 +1,5 @@
 // Zstandard frame decoding (RFC 8878), written once for a team of lanes that
-// run it together: a 64-lane workgroup on the GPU (zstd_decode.hip). The
+// run it together: a 256-lane workgroup on the GPU (zstd_decode.hip). The
 // frame, block and section headers are parsed by every lane alike (the same
 // bytes, the same branches); table descriptions are read by one lane, tables
 // are built and Huffman streams decoded by all lanes, with the tables in shared
@@ -585,7 +585,7 @@ __host__ __device__ __forceinline__ bool huf_streams(const Team& tm, ZState& z, 
   uint32_t most = 0;
   for (uint32_t i = 0; i < ns; ++i) most = z.hs[i].bits > most ? z.hs[i].bits : most;
   for (uint32_t base = 0; base < most;) {
-    // the pieces of this round: four quarters of whole 32-bit windows
+    // the pieces of this pass: four quarters of whole 32-bit windows
     const uint32_t even = ((most - base + 4 * per - 1) / (4 * per) + 31u) & ~31u;
     const uint32_t gq = even < kHufQuarterMax ? even : kHufQuarterMax;
     uint16_t m[kPerLane][3][3];

@@ -1,10 +1,10 @@
 // CPU check of the GPU zstd decoder's core (bigsmall_amd/csrc/zstd_core.h),
-// run as a one-lane team and, when built with BS_ZSTD_TEAM64, also as the GPU's
-// 64-lane team (lanes as fibers, bigsmall_amd/csrc/simt_cpu.h), against
+// run as a one-lane team and, when built with BS_ZSTD_TEAM64, also as a team of
+// BS_ZSTD_LANES lanes, 64 or the GPU's 256 (lanes as fibers, bigsmall_amd/csrc/simt_cpu.h), against
 // libzstd (the format's reference implementation). Built by
 // tests/test_zstd_core_cpu.py under AddressSanitizer and UBSan, so any read or
 // write outside the input, output or literal buffers fails the run. The
-// 64-lane team must give the one-lane team's error code and bytes on every
+// larger team must give the one-lane team's error code and bytes on every
 // frame: its lanes run one after another between barriers, so a lane that
 // reads what another writes without a barrier between them is caught.
 //   1. round trips: several data kinds x compression levels, checksum and
@@ -69,10 +69,13 @@ Bytes compress(const Bytes& in, int level, int checksum = 0, int content_size = 
 bs_zstd::ZState g_state;
 
 #ifdef BS_ZSTD_TEAM64
-// The GPU's team: 64 lanes, the workgroup barrier as sync().
+// A workgroup's team: its lanes (the GPU's has 256), the workgroup barrier as sync().
+#ifndef BS_ZSTD_LANES
+#define BS_ZSTD_LANES 64
+#endif
 struct FiberTeam {
-  static constexpr uint32_t size = 64;
-  uint32_t lane() const { return __lane_id(); }
+  static constexpr uint32_t size = BS_ZSTD_LANES;
+  uint32_t lane() const { return threadIdx.x; }
   void sync() const { __syncthreads(); }
 };
 long g_team_mismatch = 0;
@@ -109,11 +112,11 @@ int decode(const Bytes& frame, size_t cap, Bytes* out) {
       __shared__ bs_zstd::ZState z;
       uint64_t g = 0;
       const int r = bs_zstd::zstd_frames(FiberTeam{}, z, s, n, d, c, lit, g);
-      if (__lane_id() == 0) {
+      if (threadIdx.x == 0) {
         err = r;
         got = g;
       }
-    }, dim3(1), dim3(64), 0, nullptr);
+    }, dim3(1), dim3(BS_ZSTD_LANES), 0, nullptr);
     return err;
   });
   if (e64 != e || out64 != *out) ++g_team_mismatch;
@@ -212,7 +215,7 @@ int main(int argc, char** argv) {
   long team = 0;
 #ifdef BS_ZSTD_TEAM64
   team = g_team_mismatch;
-  std::printf("64-lane team differs from one lane on %ld frames\n", team);
+  std::printf("%d-lane team differs from one lane on %ld frames\n", BS_ZSTD_LANES, team);
 #endif
   std::printf("round trips %ld (failed %ld); corruptions: decoded like libzstd %ld, decoded differently %ld, "
               "decoded where libzstd refuses %ld, refused where libzstd decodes %ld, both refuse %ld\n",

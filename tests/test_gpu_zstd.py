@@ -346,8 +346,8 @@ def test_delta_roundtrip_against_safetensors_and_bs_base(tmp_path):
 
 @pytest.mark.parametrize("distinct,skew", [(2, 1.0), (16, 1.0), (40, 0.9), (256, 0.97), (24, 0.55)])
 def test_huffman_streams_of_every_length(distinct, skew):
-    """Literal sections whose streams end anywhere in a piece of the parallel Huffman decode (pieces of 32 to
-    512 bits, 16 or 64 a round): one and four streams, codes of one to eleven bits, one round and several."""
+    """Literal sections whose streams end anywhere in a piece of the parallel Huffman decode (quarters of 32 to
+    128 bits, 16 or 64 pieces a pass): one and four streams, codes of one to eleven bits, one pass and several."""
     rng = np.random.default_rng(distinct)
     p = skew ** np.arange(distinct)
     p /= p.sum()

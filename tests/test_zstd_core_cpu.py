@@ -47,3 +47,22 @@ def test_zstd_core_round_trips_and_corruptions(tmp_path):
     assert "failed 0" in r.stdout and "decoded differently 0" in r.stdout
     if team64:
         assert "64-lane team differs from one lane on 0 frames" in r.stdout
+
+
+@pytest.mark.skipif(not Path(CLANG).exists() or ctypes.util.find_library("zstd") is None,
+                    reason="needs ROCm's clang++ and libzstd")
+def test_zstd_core_as_the_gpus_256_lanes(tmp_path):
+    """The same check with the team the GPU runs, 256 lanes, on fewer corrupted frames."""
+    import ctypes
+    lib = ctypes.CDLL(ctypes.util.find_library("zstd"))._name
+    path = next((d / lib for d in map(Path, ("/usr/lib/x86_64-linux-gnu", "/usr/lib64", "/usr/lib",
+                                             "/lib/x86_64-linux-gnu")) if (d / lib).exists()), None)
+    if path is None:
+        pytest.skip(f"cannot locate {lib}")
+    exe = tmp_path / "zstd_core_check256"
+    subprocess.run([CLANG, "-O2", "-DBS_ZSTD_TEAM64", "-DBS_ZSTD_LANES=256", "-std=c++17", "-Wno-unknown-pragmas",
+                    str(ROOT / "tests/native/zstd_core_check.cpp"), str(path), "-o", str(exe)],
+                   check=True, capture_output=True, timeout=300)
+    r = subprocess.run([str(exe), "15"], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+    assert "failed 0" in r.stdout and "256-lane team differs from one lane on 0 frames" in r.stdout
