@@ -3,7 +3,7 @@ CPU under AddressSanitizer and UBSan and checked against libzstd: round trips
 over data kinds and levels -5..22, and 4,800 corrupted frames, each of which
 must decode to libzstd's bytes or be refused, with no access outside its
 buffers (tests/native/zstd_core_check.cpp). Built with ROCm's clang++, every
-frame also runs through the GPU's 64-lane team (each lane a fiber of
+frame also runs through a 64-lane team (each lane a fiber of
 bigsmall_amd/csrc/simt_cpu.h, sync() the workgroup barrier), which must give
 the one-lane team's bytes and error code on every frame; with only g++ the
 one-lane team runs alone. The GPU runs the same code (tests/test_gpu_zstd.py)."""
