@@ -257,9 +257,12 @@ class CompressedKVCache:
             L = self._blocks[layer_idx]
             ids = self._block_ids(L, layer_idx, block_ids)
             k, v = _block_outputs(len(ids), L, dev)
+            base, step = L.arena.data_ptr(), 2 * k.stride(0)
+            outp = k.data_ptr(), v.data_ptr()
             for j, bi in enumerate(ids):
-                for blocks, out in ((L.k_blocks, k), (L.v_blocks, v)):
-                    off, nb, nch, mode = blocks[bi]
-                    jobs.append(ChunkJob(L.arena.data_ptr() + off, nb, out[j].data_ptr(), L.block_elems, nch, mode))
+                # the requested rows alone: a list of the layer's every block costs more than the request
+                for blocks, out in zip((L.k, L.v), outp):
+                    off, nb, nch, mode = blocks[bi].tolist()
+                    jobs.append(ChunkJob(base + off, nb, out + j * step, L.block_elems, nch, mode))
             results.append((k, v))
         return ChunkBatch(jobs, dev), results

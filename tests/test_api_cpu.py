@@ -217,6 +217,48 @@ def test_kv_len_counts_a_layer_once_and_block_ids_are_checked():
             cache._block_ids(L, 0, bad)
 
 
+def _stub_layer(n_blocks: int, seed: int = 0):
+    """A layer of n_blocks blocks of 16 tokens whose table is made up and whose arena is empty host memory."""
+    from bigsmall_amd.kv_cache_manager import _LayerBlocks
+    rng = np.random.default_rng(seed)
+    rows = [np.stack([256 * rng.permutation(n_blocks), rng.integers(64, 4096, n_blocks),
+                      np.ones(n_blocks, np.int64), np.ones(n_blocks, np.int64)], 1) for _ in range(2)]
+    return _LayerBlocks([1, 2, 16, 8], 256, torch.zeros(256, dtype=torch.uint8), *(r.tolist() for r in rows))
+
+
+def _best_us(f, reps: int) -> float:
+    import time
+    best = 1e9
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        f()
+        best = min(best, time.perf_counter() - t0)
+    return best * 1e6
+
+
+def test_preparing_blocks_costs_by_the_request_not_by_the_layer(monkeypatch):
+    """prepare_blocks_multi reads the requested blocks' table rows only: 64 ids
+    of a layer of 4,096 blocks cost what 64 of 64 do (a list of the layer's
+    every block, made per id, would take 64 times as long), and the jobs are
+    the requested rows, K and V in turn."""
+    from bigsmall_amd import device
+    from bigsmall_amd.kv_cache_manager import CompressedKVCache
+    monkeypatch.setattr(device, "require_gpu", lambda d=None: torch.device("cpu"))
+    cache = CompressedKVCache(device="cuda")
+    cache._blocks = {0: _stub_layer(64), 1: _stub_layer(4096, 1)}
+    ids = np.random.default_rng(2).permutation(64).tolist()
+    batch, outs = cache.prepare_blocks_multi([(1, ids)])
+    L = cache._blocks[1]
+    want = []
+    for j, bi in enumerate(ids):
+        for blocks, out in zip((L.k_blocks, L.v_blocks), outs[0]):
+            off, nbytes, nch, mode = blocks[bi]
+            want.append((L.arena.data_ptr() + off, nbytes, out[j].data_ptr(), 256, nch, mode))
+    assert [(j.blob_ptr, j.blob_bytes, j.out_ptr, j.n, j.n_chunks, j.plane_mode) for j in batch.jobs] == want
+    few, many = (_best_us(lambda: cache.prepare_blocks_multi([(layer, ids)]), 20) for layer in (0, 1))
+    assert many < 4 * few, (few, many)
+
+
 @pytest.mark.parametrize("master_dtype,follower_dtype,shape", [
     (torch.float32, torch.int32, [4, 300]),          # all-zero buffers of two dtypes share one blob
     (torch.bfloat16, torch.float16, [600]),          # same 16-bit words, other dtype
