@@ -114,9 +114,8 @@ def decompress_kv_entry(data: bytes, device: str = "cuda"):
             rows.append((d.data_ptr() + pos, blen, o.data_ptr(), n, inf.n_chunks, inf.plane_mode))
         pos += (blen + 255) & ~255
     if rows:
-        t = np.array(rows, np.int64)
-        tasks, groups = chunk_tasks(t[:, 0], t[:, 1], t[:, 2], t[:, 3], t[:, 4])
-        decode_chunk_tasks(buf, d, tasks, groups, int(t[:, 5].max()), torch.cuda.current_stream(dev), "KV entry")
+        tasks, groups, max_mode = chunk_tasks(rows)
+        decode_chunk_tasks(buf, d, tasks, groups, max_mode, torch.cuda.current_stream(dev), "KV entry")
     k, v = outs
     if str(device) == "cpu":
         return k.cpu(), v.cpu()

@@ -73,6 +73,38 @@ def _block_outputs(n_blocks: int, L, dev):
     return outs[0], outs[1]
 
 
+# Requested blocks of a layer from which its task rows are made with array operations (a
+# dozen of them, whatever the count) and not one by one. MI355X, get_blocks_multi of 32
+# layers, us a call, one by one / arrays: 1 block of each 244 / 475, 4 352 / 505, 8 519 / 567,
+# 12 707 / 648, 16 843 / 686.
+FEW_BLOCKS = 10
+
+
+def _block_rows(rows: list, L: _LayerBlocks, ids: list, k, v) -> None:
+    """Append {blob, bytes, output, elements, chunks, plane mode} of each block,
+    K and V in turn, to rows. Only the requested rows of the layer's tables are
+    read: a list of its every block would cost more than the request."""
+    base, step, outp = L.arena.data_ptr(), 2 * k.stride(0), (k.data_ptr(), v.data_ptr())
+    for j, bi in enumerate(ids):
+        for blocks, out in zip((L.k, L.v), outp):
+            off, nbytes, n_chunks, mode = blocks[bi].tolist()
+            rows.append((base + off, nbytes, out + j * step, L.block_elems, n_chunks, mode))
+
+
+def _block_rows_array(L: _LayerBlocks, ids: list, k, v) -> np.ndarray:
+    """The same rows as an array, K's before V's."""
+    n = len(ids)
+    rows, at = np.empty((2, n, 6), np.int64), np.arange(n, dtype=np.int64) * (2 * k.stride(0))
+    for r, blocks, out in zip(rows, (L.k, L.v), (k, v)):
+        b = blocks[ids]
+        np.add(b[:, 0], L.arena.data_ptr(), out=r[:, 0])
+        r[:, 1] = b[:, 1]
+        np.add(at, out.data_ptr(), out=r[:, 2])
+        r[:, 3] = L.block_elems
+        r[:, 4:] = b[:, 2:]
+    return rows.reshape(-1, 6)
+
+
 class CompressedKVCache:
     """Compressed KV storage. device: where get()/get_blocks() materialise tensors."""
 
@@ -211,38 +243,32 @@ class CompressedKVCache:
         return self.get_blocks_multi([(layer_idx, block_ids)])[0]
 
     def get_blocks_multi(self, requests, stream=None):
-        """Decode the blocks of every (layer_idx, block_ids) request in one launch.
-
-        The task table is built per request with array operations, not per
-        block, and goes up with the status word in one copy: 1,024 K/V block
-        pairs took 1.87 ms with a Python loop over them, 0.18 ms of it decode."""
+        """Decode the blocks of every (layer_idx, block_ids) request in one
+        launch, whose task table goes up with the status word in one copy."""
         import torch
         from .device import chunk_tasks, decode_chunk_tasks, require_gpu
         dev = require_gpu(self.device)
-        rows, addr, outp, elems, results = [], [], [], [], []
+        few, many, results = [], [], []
         for layer_idx, block_ids in requests:
             L = self._blocks[layer_idx]
             ids = self._block_ids(L, layer_idx, block_ids)
             k, v = _block_outputs(len(ids), L, dev)
             results.append((k, v))
-            if not ids:
-                continue
-            for blocks, out in ((L.k, k), (L.v, v)):
-                rows.append(blocks[ids])
-                addr.append(rows[-1][:, 0] + L.arena.data_ptr())
-                outp.append(out.data_ptr() + 2 * out.stride(0) * np.arange(len(ids), dtype=np.int64))
-                elems.append(np.full(len(ids), L.block_elems, np.int64))
-        if rows:
-            row = np.concatenate(rows)
-            tasks, groups = chunk_tasks(np.concatenate(addr), row[:, 1], np.concatenate(outp), np.concatenate(elems),
-                                        row[:, 2])
+            if len(ids) < FEW_BLOCKS:
+                _block_rows(few, L, ids, k, v)
+            else:
+                many.append(_block_rows_array(L, ids, k, v))
+        if few or many:
+            if many:
+                many.append(np.array(few, np.int64).reshape(-1, 6))
+            tasks, groups, max_mode = chunk_tasks(np.concatenate(many) if many else few)
             s = stream if stream is not None else torch.cuda.current_stream(dev)
             if stream is not None:        # the outputs' memory and the arenas are the current stream's
                 s.wait_stream(torch.cuda.current_stream(dev))
             nbytes = 256 + tasks.nbytes
             host = torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
             decode_chunk_tasks(host.numpy(), torch.empty(nbytes, dtype=torch.uint8, device=dev), tasks, groups,
-                               int(row[:, 3].max()), s, "KV blocks")
+                               max_mode, s, "KV blocks")
         return [(k.contiguous(), v.contiguous()) for k, v in results]
 
     def prepare_blocks_multi(self, requests):
@@ -252,17 +278,11 @@ class CompressedKVCache:
         import torch
         from .device import ChunkBatch, ChunkJob, require_gpu
         dev = require_gpu(self.device)
-        jobs, results = [], []
+        rows, results = [], []
         for layer_idx, block_ids in requests:
             L = self._blocks[layer_idx]
             ids = self._block_ids(L, layer_idx, block_ids)
             k, v = _block_outputs(len(ids), L, dev)
-            base, step = L.arena.data_ptr(), 2 * k.stride(0)
-            outp = k.data_ptr(), v.data_ptr()
-            for j, bi in enumerate(ids):
-                # the requested rows alone: a list of the layer's every block costs more than the request
-                for blocks, out in zip((L.k, L.v), outp):
-                    off, nb, nch, mode = blocks[bi].tolist()
-                    jobs.append(ChunkJob(base + off, nb, out + j * step, L.block_elems, nch, mode))
+            _block_rows(rows, L, ids, k, v)
             results.append((k, v))
-        return ChunkBatch(jobs, dev), results
+        return ChunkBatch([ChunkJob(*r) for r in rows], dev), results

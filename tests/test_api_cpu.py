@@ -259,6 +259,75 @@ def test_preparing_blocks_costs_by_the_request_not_by_the_layer(monkeypatch):
     assert many < 4 * few, (few, many)
 
 
+@pytest.mark.parametrize("layers,blocks,odd", [(1, 1, False), (8, 1, False), (32, 1, False), (32, 2, False), (32, 9, False),
+                                               (3, 10, False), (4, 11, True), (2, 64, True), (8, 64, False)])
+def test_block_requests_build_the_same_tasks_as_a_loop_and_no_slower(monkeypatch, layers, blocks, odd):
+    """get_blocks_multi's task table holds the task of every requested K and V
+    block once (few blocks of a layer are added one by one, many by array
+    operations; odd: a block that is no multiple of 8 elements, whose outputs
+    are strided), and building it, with the upload and launch stubbed out,
+    takes no longer than a loop of one job per block does."""
+    from bigsmall_amd import device
+    from bigsmall_amd.device import ChunkBatch, ChunkJob
+    from bigsmall_amd.kv_cache_manager import CompressedKVCache, _block_outputs
+    cpu, empty, got = torch.device("cpu"), torch.empty, []
+    monkeypatch.setattr(device, "require_gpu", lambda d=None: cpu)
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: None)
+    monkeypatch.setattr(device, "decode_chunk_tasks",
+                        lambda buf, d_buf, tasks, groups, max_mode, stream, what: got.append((tasks, groups, max_mode)))
+    cache = CompressedKVCache(device="cuda")
+    for i in range(layers):
+        L = cache._blocks[i] = _stub_layer(256, i)
+        if odd:
+            L.block_shape, L.block_elems = [1, 2, 13, 7], 182
+        L.k[:, 2:], L.v[:, 2:] = (3, 1), (3, 2)                     # three chunks a block; V compact
+    rng = np.random.default_rng(layers)
+    requests = [(i, rng.integers(0, 256, blocks).tolist()) for i in range(layers)]
+
+    def loop():
+        jobs, outs = [], []
+        for i, ids in requests:
+            L = cache._blocks[i]
+            k, v = _block_outputs(len(ids), L, cpu)
+            base = L.arena.data_ptr()
+            for j, bi in enumerate(cache._block_ids(L, i, ids)):
+                for table, out in ((lists[i][0], k), (lists[i][1], v)):
+                    off, nb, nch, mode = table[bi]
+                    jobs.append(ChunkJob(base + off, nb, out[j].data_ptr(), L.block_elems, nch, mode))
+            outs.append((k, v))
+        ChunkBatch(jobs, cpu)
+        return jobs, [(k.contiguous(), v.contiguous()) for k, v in outs]
+
+    lists = {i: (cache._blocks[i].k_blocks, cache._blocks[i].v_blocks) for i in range(layers)}
+    outputs = {}
+
+    def recorded(n, L, dev):                                        # both sides with the same output addresses
+        key = (id(L), n)
+        if key not in outputs:
+            outputs[key] = _block_outputs(n, L, dev)
+        return outputs[key]
+
+    with monkeypatch.context() as m:
+        m.setattr("bigsmall_amd.kv_cache_manager._block_outputs", recorded)
+        cache.get_blocks_multi(requests)
+    tasks, groups, max_mode = got[-1]
+    want = set()
+    for i, ids in requests:
+        L = cache._blocks[i]
+        for out, table in zip(recorded(len(ids), L, cpu), lists[i]):
+            for j, bi in enumerate(ids):
+                off, nb, nch, _ = table[bi]
+                want.add((L.arena.data_ptr() + off, nb, out[j].data_ptr(), L.block_elems, nch))
+    assert {tuple(t.tolist()[:4]) + (int(t["n_chunks"]),) for t in tasks} == want
+    assert len(tasks) == 2 * layers * blocks and max_mode == 2
+    assert tasks["wg_begin"].tolist() == list(range(len(tasks))) and groups == len(tasks)
+    reps = 30
+    ours, theirs = _best_us(lambda: cache.get_blocks_multi(requests), reps), _best_us(loop, reps)
+    print(f"{layers} x {blocks}: {ours:.0f} us, loop {theirs:.0f} us")
+    assert ours < 1.3 * theirs + 15, (ours, theirs)
+
+
 @pytest.mark.parametrize("master_dtype,follower_dtype,shape", [
     (torch.float32, torch.int32, [4, 300]),          # all-zero buffers of two dtypes share one blob
     (torch.bfloat16, torch.float16, [600]),          # same 16-bit words, other dtype
