@@ -38,13 +38,14 @@ def compress_kv_entry(keys, values) -> bytes:
     tensors use the host encoder (the reference copies to the host and encodes
     there, kv_cache.py:28-38)."""
     import torch
+    from ..device import pinned_bytes
     if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
         raise ValueError("compress_kv_entry requires BF16 keys and values")
     if keys.is_cuda and values.is_cuda and keys.numel() and values.numel():
         # only the blobs come back (the encoder's arena holds a worst case for
         # each), through pinned memory
         arena, spans = bf16_chunked.encode_device([keys, values], steps=KV_STEPS, compact=False)
-        host = torch.empty(sum(n for _, n in spans), dtype=torch.uint8, pin_memory=True)
+        host = pinned_bytes(sum(n for _, n in spans))
         blobs, pos = [], 0
         for o, n in spans:
             host[pos:pos + n].copy_(arena[o:o + n], non_blocking=True)
@@ -93,7 +94,7 @@ def parse_kv_entry(data: bytes) -> list[tuple[list[int], int, int, int]]:
 def decompress_kv_entry(data: bytes, device: str = "cuda"):
     """Inverse of compress_kv_entry: (keys, values) as bf16 tensors on `device`."""
     import torch
-    from ..device import TASK_DTYPE, chunk_tasks, decode_chunk_tasks, require_gpu
+    from ..device import TASK_DTYPE, chunk_tasks, decode_chunk_tasks, pinned_bytes, require_gpu
     parts = parse_kv_entry(data)
     dev = require_gpu(device if str(device) != "cpu" else None)
     # one pinned buffer and one copy: status word, task table (its own 256 bytes), K's and V's blobs
@@ -101,7 +102,7 @@ def decompress_kv_entry(data: bytes, device: str = "cuda"):
     assert 256 + 2 * TASK_DTYPE.itemsize <= pos
     total = pos + sum((b + 255) & ~255 for _, _, _, b in parts)
     d = torch.empty(total, dtype=torch.uint8, device=dev)
-    buf = torch.empty(total, dtype=torch.uint8, pin_memory=True).numpy()
+    buf = pinned_bytes(total).numpy()
     outs, rows = [], []
     for shape, n, off, blen in parts:
         o = torch.empty(shape if all(s > 0 for s in shape) else [n], dtype=torch.bfloat16, device=dev)

@@ -52,6 +52,12 @@ def upload_bytes(data, device, align: int = 256):
     return out
 
 
+def pinned_bytes(n: int):
+    """A pinned host uint8 tensor of n bytes (on the host whatever torch's default device is)."""
+    import torch
+    return torch.empty(n, dtype=torch.uint8, device="cpu", pin_memory=True)
+
+
 def upload_bytes_async(data, device, stream=None):
     """upload_bytes through pinned staging with a non-blocking copy on
     `stream` (the current stream if None): the host does not wait for the
@@ -62,7 +68,7 @@ def upload_bytes_async(data, device, stream=None):
     arr = np.frombuffer(data, np.uint8) if not isinstance(data, np.ndarray) else data.view(np.uint8).reshape(-1)
     out = torch.empty(len(arr), dtype=torch.uint8, device=device)
     if len(arr):
-        host = torch.empty(len(arr), dtype=torch.uint8, pin_memory=True)
+        host = pinned_bytes(len(arr))
         host.numpy()[:] = arr
         with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
             out.copy_(host, non_blocking=True)

@@ -42,7 +42,7 @@ from .codecs import _refstreams
 from .codecs import bf16_chunked
 from .codecs import zstd_gpu
 from .container import tensor_numel
-from .device import ChunkBatch, ChunkJob, StatusWord, require_gpu
+from .device import ChunkBatch, ChunkJob, StatusWord, pinned_bytes, require_gpu
 from .exceptions import BigSmallVersionError
 from .formats import torch_dtype
 
@@ -174,7 +174,7 @@ class GroupDecoder:
             ev.synchronize()              # the copy that last read this buffer has finished
         buf = self._pinned[i]
         if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, pin_memory=True)
+            buf = pinned_bytes(max(nbytes, 1 << 20))
             self._pinned[i] = buf
         return i, buf
 

@@ -246,7 +246,7 @@ class CompressedKVCache:
         """Decode the blocks of every (layer_idx, block_ids) request in one
         launch, whose task table goes up with the status word in one copy."""
         import torch
-        from .device import chunk_tasks, decode_chunk_tasks, require_gpu
+        from .device import chunk_tasks, decode_chunk_tasks, pinned_bytes, require_gpu
         dev = require_gpu(self.device)
         few, many, results = [], [], []
         for layer_idx, block_ids in requests:
@@ -264,10 +264,11 @@ class CompressedKVCache:
             tasks, groups, max_mode = chunk_tasks(np.concatenate(many) if many else few)
             s = stream if stream is not None else torch.cuda.current_stream(dev)
             if stream is not None:        # the outputs' memory and the arenas are the current stream's
+                if not isinstance(s, torch.cuda.Stream):        # any object with a cuda_stream handle
+                    s = torch.cuda.ExternalStream(int(s.cuda_stream), device=dev)
                 s.wait_stream(torch.cuda.current_stream(dev))
             nbytes = 256 + tasks.nbytes
-            host = torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
-            decode_chunk_tasks(host.numpy(), torch.empty(nbytes, dtype=torch.uint8, device=dev), tasks, groups,
+            decode_chunk_tasks(pinned_bytes(nbytes).numpy(), torch.empty(nbytes, dtype=torch.uint8, device=dev), tasks, groups,
                                max_mode, s, "KV blocks")
         return [(k.contiguous(), v.contiguous()) for k, v in results]
 

@@ -603,3 +603,28 @@ def test_kv_block_requests_in_one_table(tmp_path, block_shape):
                 assert out.shape == (len(ids), heads, tokens, dim) and out.is_contiguous()
                 for j, b in enumerate(ids):
                     assert torch.equal(out[j].view(torch.int16), whole[:, b * tokens:(b + 1) * tokens].contiguous().view(torch.int16))
+
+
+def test_kv_calls_under_a_cuda_default_device_and_on_a_foreign_stream():
+    """The KV cache's calls run with torch's default device set to the GPU (their
+    pinned staging stays on the host), and get_blocks_multi takes any stream
+    object that has a cuda_stream handle."""
+    import types
+
+    from bigsmall_amd.kv_cache_manager import CompressedKVCache
+    g = torch.Generator().manual_seed(2)
+    k, v = ((torch.randn(2, 96, 64, generator=g) * 0.5).to(torch.bfloat16).cuda() for _ in range(2))
+    cache = CompressedKVCache(device="cuda")
+    want = [(t.view(2, 6, 16, 64).transpose(0, 1)[[4, 1]], t) for t in (k, v)]
+    with torch.device("cuda"):
+        for where in ("cuda", "cpu"):
+            _say(f"[kv] default device cuda, K and V on {where}")
+            cache.set(0, k.to(where), v.to(where))
+            cache.set_blocks(0, k.to(where), v.to(where), block_tokens=16)
+            for out, blocks, (b, whole) in zip(cache.get(0), cache.get_blocks(0, [4, 1]), want):
+                assert torch.equal(out, whole) and torch.equal(blocks, b)
+    own = torch.cuda.Stream()
+    _say("[kv] a stream object of another kind")
+    out = cache.get_blocks_multi([(0, [4, 1])], stream=types.SimpleNamespace(cuda_stream=own.cuda_stream))
+    for blocks, (b, _) in zip(out[0], want):
+        assert torch.equal(blocks, b)
