@@ -142,11 +142,11 @@ __global__ __launch_bounds__(kMantThreads) void mant_kernel(const bs_mant_bucket
 // buckets share a table (lane_chains, below).
 //
 // A wavefront's chain keeps its state in a scalar register and its symbols
-// spread over the lanes (serial_chain); the lanes also load the word stream 1 KB
-// at a time into an LDS byte ring one segment ahead of use, hold a 64-word
-// window of it, and keep the symbols of 64 steps (lane j: step j) for one
-// coalesced store. The SE chain writes sign<<15 | exp<<7 of
-// every element and counts the exponents of each tile of kTile symbols of its
+// spread over the lanes (serial_chain), or, with many symbols, reads a table
+// (table_chain); the lanes also load the word stream 1 KB at a time into an LDS
+// byte ring one segment ahead of use, hold a 64-word window of it, and keep the
+// symbols of 64 steps (lane j: step j) for one coalesced store. The SE chain
+// writes sign<<15 | exp<<7 of every element and counts the exponents of each tile of kTile symbols of its
 // stream; the mantissa chains, which do not depend on it, run at the same time
 // in other workgroups and write their bucket's mantissas in bucket order. Two
 // parallel passes then give every element its position in its (stream,
@@ -223,6 +223,56 @@ __device__ __forceinline__ void tile_count_end(GLB uint32_t* ghist, uint32_t lan
   for (uint64_t i = ((uint64_t)n + kTile - 1) / kTile * 256u + lane; i < (uint64_t)tps * 256u; i += kWave) ghist[i] = 0;
 }
 
+__device__ __forceinline__ uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t uni64(uint64_t v) {
+  return (uint64_t)uni32((uint32_t)v) | ((uint64_t)uni32((uint32_t)(v >> 32)) << 32);
+}
+
+// A chain's words: its bytes go through the wave's LDS ring, loaded a segment
+// ahead of use, into a window of 64 words: lane l of `win` holds word base + l
+// (past the stream: the tail word). A step takes at most one word, so a window
+// moved on when the chain has taken kHalf of it lasts another kHalf steps.
+constexpr uint32_t kHalf = 32;           // steps between looks at the window
+struct WordWindow {
+  const GLB uint8_t* A;                  // the stream starts at A + s_off, A 16-byte aligned
+  uint32_t s_off, n_words, tail_word;
+  uint64_t e_off;
+  LDS uint8_t* ring;
+  uint64_t landed = 0;                   // stream bytes [.., landed) are in the ring (relative to A)
+  bool inflight = false;                 // segment `landed / kSegB` is being loaded into `seg`
+  u32x4 seg = {0u, 0u, 0u, 0u};
+  uint32_t base = 0, win = 0;
+  __device__ __forceinline__ WordWindow(const GLB uint8_t* words, uint32_t n, uint32_t tail, LDS uint8_t* r)
+      : n_words(n), tail_word(tail & 0xFFFFu), ring(r) {
+    const uint64_t wa = uni64((uint64_t)words);
+    A = (const GLB uint8_t*)(wa & ~15ull);
+    s_off = (uint32_t)(wa & 15u);
+    e_off = s_off + 2ull * n_words;
+  }
+  // moves the window on by `taken` words
+  __device__ __forceinline__ void move(uint32_t taken, uint32_t lane) {
+    base = uni32(base + taken);
+    const uint64_t consumed = s_off + 2ull * base;
+    if (inflight) {
+      seg_land(ring, landed / kSegB, lane, seg);
+      landed += kSegB;
+      inflight = false;
+    }
+    while (landed < e_off && landed < consumed + 2u * kWave + 2u) {
+      seg_land(ring, landed / kSegB, lane, seg_block(A, landed / kSegB, lane, s_off, e_off));
+      landed += kSegB;
+    }
+    if (landed < e_off && landed + kSegB <= consumed + kRingB) {
+      seg = seg_block(A, landed / kSegB, lane, s_off, e_off);
+      inflight = true;
+    }
+    wave_sync();
+    const uint32_t b = s_off + 2u * (base + lane);
+    win = (uint32_t)ring[b & (kRingB - 1u)] | ((uint32_t)ring[(b + 1u) & (kRingB - 1u)] << 8);
+    win = base + lane < n_words ? win : tail_word;
+  }
+};
+
 // Decode one chain of n symbols with the symbols spread over the lanes: lane l
 // holds symbols l*R .. l*R + R-1 (in slot order: f and cf of each), and no table
 // is read. A step forms in every lane the state its symbol would give,
@@ -250,11 +300,6 @@ __device__ __forceinline__ void tile_count_end(GLB uint32_t* ghist, uint32_t lan
 // and an initial state below L, which no encoder writes, is reported as a
 // corrupt stream. A corrupt stream that runs out of words shifts in its tail
 // word (zero when it has none) and fails the end-of-stream check.
-__device__ __forceinline__ uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ uint64_t uni64(uint64_t v) {
-  return (uint64_t)uni32((uint32_t)v) | ((uint64_t)uni32((uint32_t)(v >> 32)) << 32);
-}
-
 // A symbol of a chain's table in LDS: f | cf << 16, and its output (SE: the
 // word sign<<15 | exp<<7; mantissa: the 7 bits).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -296,22 +341,13 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
                                              GLB uint8_t* __restrict__ out, uint32_t stride, LDS uint32_t* hist,
                                              GLB uint32_t* ghist, uint32_t tps, int32_t* status) {
   constexpr uint32_t kLog = SE ? 12u : 10u, kTop = 32u - kLog;
-  constexpr uint32_t kHalf = 32;       // steps between looks at the word window
   // the descriptor's fields are the same in every lane: say so, so that the
   // chain's state and word position stay scalar
   n_words = uni32(n_words);
   tail = uni32(tail);
   n = uni32(n);
   const uint32_t lane = __lane_id();
-  const uint64_t wa = uni64((uint64_t)words);
-  const GLB uint8_t* A = (const GLB uint8_t*)(wa & ~15ull);
-  const uint32_t s_off = (uint32_t)(wa & 15u);
-  const uint64_t e_off = s_off + 2ull * n_words;
   const uint32_t n_eff = n_words + ((tail >> 16) & 1u);
-  const uint32_t tail_word = tail & 0xFFFFu;
-  uint64_t landed = 0;        // stream bytes [.., landed) are in the ring (relative to A)
-  bool inflight = false;      // segment `landed / kSegB` is being loaded into `seg`
-  u32x4 seg = {0u, 0u, 0u, 0u};
   uint32_t x = uni32(x0);
   if (x < kL) {
     if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
@@ -320,31 +356,12 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
   if (SE) tile_count_begin(hist, lane);
   LaneSyms<R, SE> S;
   S.load(syms, live, lane);
-  // Word window: lane l of `win` holds word base + l (past the stream: the tail
-  // word); the next word is lane `at`'s. A step takes at most one word, so a
-  // window moved on when `at` has reached kHalf lasts another kHalf steps.
-  uint32_t base = 0, at = kWave, win = 0;
+  WordWindow W(words, n_words, tail, ring);
+  uint32_t at = kWave, win = 0;          // the next word is lane `at`'s; kWave: no window yet
   auto window = [&]() {
-    base = uni32(base + (at == kWave ? 0u : at));
+    W.move(at == kWave ? 0u : at, lane);
     at = 0;
-    const uint64_t consumed = s_off + 2ull * base;
-    if (inflight) {
-      seg_land(ring, landed / kSegB, lane, seg);
-      landed += kSegB;
-      inflight = false;
-    }
-    while (landed < e_off && landed < consumed + 2u * kWave + 2u) {
-      seg_land(ring, landed / kSegB, lane, seg_block(A, landed / kSegB, lane, s_off, e_off));
-      landed += kSegB;
-    }
-    if (landed < e_off && landed + kSegB <= consumed + kRingB) {
-      seg = seg_block(A, landed / kSegB, lane, s_off, e_off);
-      inflight = true;
-    }
-    wave_sync();
-    const uint32_t b = s_off + 2u * (base + lane);
-    win = (uint32_t)ring[b & (kRingB - 1u)] | ((uint32_t)ring[(b + 1u) & (kRingB - 1u)] << 8);
-    win = base + lane < n_words ? win : tail_word;
+    win = W.win;
   };
   uint32_t acc = 0;            // lane j: the symbol index (lane * R + r) of step j of the batch
   // One step: x becomes the next state, and lane j of acc takes the symbol's
@@ -431,30 +448,9 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
                    [begin] "v"(S.begin[R - 1]), [win] "v"(win), [log] "i"(kLog), [top] "i"(kTop), [step] "i"(j)       \
                  : "vcc", "scc");                                                                                     \
   }
-  auto step_many = [&](uint32_t j) {
-    const uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)win, (int)at), t = (x << kTop) + S.first;
-    const uint64_t hit = __ballot(t <= S.last);
-    uint32_t c = (uint32_t)__mul24(S.nf[0], (int)(x >> kLog)) + (x - S.cf[0]), sym = lane * R;
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      const uint32_t cr = (uint32_t)__mul24(S.nf[r], (int)(x >> kLog)) + (x - S.cf[r]);
-      const bool ge = t >= S.begin[r];
-      c = ge ? cr : c;
-      sym = ge ? lane * R + r : sym;
-    }
-    const bool low = c < kL;
-    const uint64_t need = __ballot(low);
-    const uint32_t y = low ? (c << 16) | w : c, l = (uint32_t)__builtin_ctzll(hit);
-    x = (uint32_t)__builtin_amdgcn_readlane((int)y, (int)l);
-    at += (uint32_t)(need >> (l & 63u)) & 1u;
-    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)sym, (int)l);
-    // (a select on lane == j would hold the batch's 64 lane masks in registers)
-    asm volatile("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(acc) : "s"(o), "i"(j));
-  };
-#define BS_STEP(j)                       \
-  if constexpr (R == 1) BS_STEP1(j)      \
-  else if constexpr (R == 2) BS_STEP2(j) \
-  else step_many(j)
+#define BS_STEP(j)                  \
+  if constexpr (R == 1) BS_STEP1(j) \
+  else BS_STEP2(j)
 #endif
   auto settle = [&]() {
     x = uni32(x);
@@ -498,7 +494,79 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
 #undef BS_STEP
   if (SE) tile_count_end(ghist, lane, n, tps);
   if (at == kWave) at = 0;                               // an empty chain never opened its window
-  if (x != kL || base + at != n_eff) {
+  if (x != kL || W.base + at != n_eff) {
+    if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
+  }
+}
+
+// The SE chain of a tensor with more than 128 live symbols (a checkpoint's weights
+// have 60 or so), of which a lane would hold four or more: each of those costs a
+// step five instructions more in every lane, a table read costs one LDS latency. The table is the task's own, in LDS as 4-byte entries
+// {f | (slot - cf) << 13} beside the slots' output words, shared by the
+// workgroup's chains. The state and the word position stay in vector registers,
+// the same in every lane, so that no step waits for a scalar register; the next
+// word comes by ds_bpermute as soon as its position is known, under the next table
+// read; a step's slot goes to its place in the wave's stage, which lane j reads
+// after 64 steps. MI355X, 250 symbols: 54 ns a step on one chain (132 with eight symbols
+// per lane), 70 with 128 chains (146); held by the lanes, 120 symbols take 45 and 59.
+__device__ __forceinline__ void table_chain(const GLB uint8_t* words, uint32_t n_words, uint32_t tail, uint32_t x0,
+                                            uint32_t n, const LDS uint32_t* tbl, const LDS uint16_t* slot_words,
+                                            LDS uint16_t* stage, LDS uint8_t* ring, GLB uint16_t* __restrict__ out,
+                                            uint32_t stride, LDS uint32_t* hist, GLB uint32_t* ghist, uint32_t tps,
+                                            int32_t* status) {
+  n_words = uni32(n_words);
+  tail = uni32(tail);
+  n = uni32(n);
+  const uint32_t lane = __lane_id();
+  const uint32_t n_eff = n_words + ((tail >> 16) & 1u);
+  if (uni32(x0) < kL) {
+    if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
+    return;
+  }
+  tile_count_begin(hist, lane);
+  WordWindow W(words, n_words, tail, ring);
+  uint32_t x = x0, at4 = 0, w = 0;       // at4: 4 * the next word's lane
+  auto window = [&]() {
+    W.move(uni32(at4) >> 2, lane);
+    at4 = 0;
+    w = (uint32_t)__builtin_amdgcn_ds_bpermute(0, (int)W.win);
+  };
+  window();
+  BS_OPAQUE(x);
+  auto step = [&](uint32_t j) {
+    const uint32_t slot = x & 4095u, e = tbl[slot];
+    const uint32_t c = __umul24(e & 0x1FFFu, x >> 12) + (e >> 13);
+    *(volatile LDS uint16_t*)(stage + j) = (uint16_t)slot;
+#ifdef BS_SIMT_CPU     // an emulated exchange costs 64 fiber switches: one where a word is taken
+    x = c < kL ? (c << 16) | (uint32_t)__builtin_amdgcn_readlane((int)W.win, (int)(at4 >> 2)) : c;
+    at4 += c < kL ? 4u : 0u;
+#else
+    x = c < kL ? (c << 16) | w : c;
+    at4 += c < kL ? 4u : 0u;
+    BS_OPAQUE(x);
+    BS_OPAQUE(at4);
+    w = (uint32_t)__builtin_amdgcn_ds_bpermute((int)at4, (int)W.win);
+#endif
+  };
+  for (uint32_t i0 = 0; i0 < n; i0 += kWave) {
+    const uint32_t cnt = min((uint32_t)kWave, n - i0);
+    for (uint32_t h0 = 0; h0 < cnt; h0 += kHalf) {
+      if (uni32(at4) >= 4u * kHalf) window();
+      if (cnt - h0 >= kHalf) {
+#pragma unroll
+        for (uint32_t j = 0; j < kHalf; ++j) step(h0 + j);
+      } else {
+        for (uint32_t j = h0; j < cnt; ++j) step(j);
+      }
+    }
+    wave_sync();
+    const uint32_t word = slot_words[stage[lane] & 4095u];
+    if (lane < cnt) out[(uint64_t)(i0 + lane) * stride] = (uint16_t)word;
+    tile_count(hist, ghist, word, lane, i0, cnt, n);
+    wave_sync();
+  }
+  tile_count_end(ghist, lane, n, tps);
+  if (uni32(x) != kL || W.base + (uni32(at4) >> 2) != n_eff) {
     if (lane == 0) flag(status, BS_DEV_ERR_STREAM);
   }
 }
@@ -723,9 +791,11 @@ constexpr uint32_t kSeSyms = 512, kMantSyms = 128;
 constexpr uint32_t kSymB = kSeSyms * 8;   // one SE symbol list, or kSerWaves mantissa lists
 static_assert(kSerWaves * kMantSyms <= kSeSyms, "mantissa lists exceed the symbol area");
 constexpr uint32_t kHistB = 256 * 4;   // per SE chain: the exponent counts of its current tile
-// 48 KB: rings | symbols | tile counts (16 KB), or the lane-wise chains' tables and rings
+constexpr uint32_t kTblOff = kSerWaves * kRingB + kSymB + kSerWaves * kHistB;
+// 48 KB: rings | symbols | tile counts (16 KB) | table_chain's table, output words and stages
+// (24.5 KB), or the lane-wise chains' tables and rings
 constexpr uint32_t kSerLds = kSerWaves * kLaneB;
-static_assert(kSerLds >= kSerWaves * kRingB + kSymB + kSerWaves * kHistB, "chain LDS");
+static_assert(kSerLds >= kTblOff + 4096 * 6 + kSerWaves * kWave * 2, "chain LDS");
 
 __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_task* __restrict__ tasks,
                                                                    uint32_t n_tasks, bs_ref_task single,
@@ -764,6 +834,16 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
       off = e.x >> 13;
       o = (((e.y >> 8) & 1u) << 15) | ((e.y & 0xFFu) << 7);
     });
+    const bool table = live > 128;                        // uniform over the workgroup
+    LDS uint32_t* tbl = (LDS uint32_t*)(smem + kTblOff);
+    LDS uint16_t* slot_words = (LDS uint16_t*)(smem + kTblOff + 4096 * 4);
+    if (table) {
+      for (uint32_t i = tid; i < 4096; i += kSerWaves * kWave) {
+        const u32x2 e = t[i];
+        tbl[i] = e.x;
+        slot_words[i] = (uint16_t)((((e.y >> 8) & 1u) << 15) | ((e.y & 0xFFu) << 7));
+      }
+    }
     __syncthreads();
     if (c >= count) return;
     const bs_se_stream S = T.streams[c];
@@ -779,9 +859,12 @@ __global__ __launch_bounds__(kSerWaves * kWave) void serial_kernel(const bs_ref_
       serial_chain<decltype(r)::value, true>((const GLB uint8_t*)S.words, S.n_words, S.tail, S.x0, S.n, syms, live, ring,
                                              (GLB uint8_t*)(T.out + S.first), S.stride, hist, ghist, tps, status);
     };
-    if (live <= 64) run(std::integral_constant<int, 1>{});
-    else if (live <= 128) run(std::integral_constant<int, 2>{});
-    else run(std::integral_constant<int, 8>{});
+    if (table)
+      table_chain((const GLB uint8_t*)S.words, S.n_words, S.tail, S.x0, S.n, tbl, slot_words,
+                  (LDS uint16_t*)(smem + kTblOff + 4096 * 6) + wave * kWave, ring, (GLB uint16_t*)(T.out + S.first), S.stride,
+                  hist, ghist, tps, status);
+    else if (live <= 64) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
   } else if (lanes) {
     if ((uint64_t)c * kWave >= count) return;
     lane_chains(T.buckets, T.n_buckets, c * kWave, T.mant_tables, T.n_tables, T.n_out, mant,

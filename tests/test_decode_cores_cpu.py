@@ -137,6 +137,8 @@ def _ref_inputs(rng):
     hz = _bf16(rng.standard_normal(800) * 0.02)
     hz[rng.permutation(hz.size)[:400]] = 0
     yield "bf16_se_tans", hz, oracle.tans_encode
+    # more than 128 live sign/exponent symbols: SE chains over a table in LDS
+    yield "bf16_parallel_v1", rng.integers(0, 65536, 900).astype(np.uint16), lambda w: oracle.par1_encode(w, 3)
 
 
 def _write_cases(path: Path, n_bsck: int, n_ref: int) -> dict:

@@ -248,9 +248,9 @@ def test_serial_batch_rejects_inconsistent_task(gpu):
 @pytest.mark.parametrize("live", [1, 2, 63, 64, 65, 128, 129, 512])
 @pytest.mark.parametrize("codec", ["bf16_parallel_v1", "bf16_se_tans", "bf16_se_single_kernel"])
 def test_chain_symbol_counts(gpu, codec, live):
-    """Wave-serial chains hold 1, 2 or 8 sign/exponent symbols per lane: live symbol
-    counts on both sides of each line, one symbol of frequency 4096 among them, and
-    a last batch of fewer than 64 steps."""
+    """Wave-serial chains hold 1 or 2 sign/exponent symbols per lane, or read a table
+    from 129 on: live symbol counts on both sides of each line, one symbol of
+    frequency 4096 among them, and a last batch of fewer than 64 steps."""
     rng = np.random.default_rng(live)
     n = (1 << 16) + 37
     se = np.sort(rng.permutation(512)[:live])
@@ -258,6 +258,37 @@ def test_chain_symbol_counts(gpu, codec, live):
     w = ((se[rng.permutation(pick)] << 7) | rng.integers(0, 128, n)).astype(np.uint16)
     _say(f"[ref] {codec} with {live} live symbols")
     assert _decode(codec, CODECS[codec][0](w), n) == w.tobytes()
+
+
+def test_chains_of_many_symbols_cost_no_multiple(gpu):
+    """A chain of 250 symbols, which reads a table, takes at most 1.8 times as
+    long as one of 120, held by the lanes (1.2 measured; eight symbols per lane
+    took 2.9)."""
+    from bigsmall_amd.codecs import _refstreams
+    from bigsmall_amd.device import StatusWord, upload_bytes
+    torch = gpu
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(9)
+    n, ms = 1 << 15, {}
+    for live in (120, 250):
+        w = ((rng.integers(0, live, n) << 7) | rng.integers(0, 128, n)).astype(np.uint16)
+        blob = oracle.tans_encode(w)
+        d_blob, out, st = upload_bytes(blob, dev), torch.empty(n, dtype=torch.int16, device=dev), StatusWord(dev)
+        launch = _refstreams.RefLaunch(_refstreams.PARSERS["bf16_se_tans"](blob, n), d_blob.data_ptr(), dev,
+                                       out.data_ptr())
+        _say(f"[ref] chain of {live} symbols")
+        times = []
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            launch.launch(out.data_ptr(), st.ptr, torch.cuda.current_stream(dev).cuda_stream)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        st.check("bf16_se_tans")
+        assert out.cpu().numpy().tobytes() == w.tobytes()
+        ms[live] = min(times)
+    assert ms[250] < 1.8 * ms[120], ms
 
 
 @pytest.mark.parametrize("streams", [8, 31, 32, 33, 64, 100, 256])
