@@ -1404,23 +1404,6 @@ inline uint32_t groups_for(uint32_t n_chunks) { return (n_chunks + kWaves - 1) /
 
 std::atomic<uint64_t> g_lds_plain{0}, g_lds_compact{0};   // devices configured, one bit each
 
-// Compute units of the current device, asked once per device (devices 0..63);
-// 2^32-1 when unknown, which marks no workgroup as the younger of its CU's two.
-std::atomic<uint32_t> g_cus[64];
-uint32_t device_cus() {
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0xFFFFFFFFu;
-  uint32_t v = g_cus[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      return 0xFFFFFFFFu;
-    v = (uint32_t)n;
-    g_cus[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
-}
-
 // log2 of the workgroups that share the 8 chunks of one group of the tasks'
 // numbering. A chunk is a serial chain of steps, so a launch with fewer groups
 // than CUs is bound by the step's latency and by the waves that share a CU's
@@ -1442,7 +1425,7 @@ static_assert((kWaves & (kWaves - 1)) == 0, "every spread divides the waves of a
 
 int launch(const bs_chunk_task* tasks, uint32_t n_tasks, const bs_chunk_task& single, uint32_t groups,
            uint32_t max_mode, int32_t* status, void* stream) {
-  const uint32_t first_round = device_cus();
+  const uint32_t first_round = bs_internal::device_cus();   // 2^32-1: no workgroup is the younger of its CU's two
   const uint32_t spread = spread_for(groups, first_round);
   if (max_mode >= 2) {
     bs_internal::ensure_lds_limit((const void*)bsck_decode_kernel<true>, kLds, g_lds_compact);

@@ -3,11 +3,14 @@
 // frame, block and section headers are parsed by every lane alike (the same
 // bytes, the same branches); table descriptions are read by one lane, tables
 // are built and Huffman streams decoded by all lanes, with the tables in shared
-// memory; literal and match copies are spread over all lanes.
+// memory; long copies are spread over all lanes, short sequences run by the
+// leading ones.
 //
 // A Team provides lane() (0 .. size-1), size and sync() (a barrier that also
 // makes every lane's earlier global and shared-memory writes visible to the
-// team).
+// team), and its leading lanes, 0 .. lead_size-1 (one wavefront on the GPU):
+// leads() (true in them, the same in a whole wavefront) and lead_sync(), the
+// same among them alone.
 //
 // Every read of the input is bounds-checked; malformed input ends the task
 // with an error code, never with an out-of-bounds access. Not supported:
@@ -26,6 +29,8 @@ constexpr uint32_t kLLMax = 35, kMLMax = 52, kOFMax = 31;
 constexpr uint32_t kStageBytes = 24u << 10;    // compressed blocks up to this size are read from shared memory
 constexpr uint32_t kHufGroups = 64;            // pieces of a literal section's streams decoded side by side
 constexpr uint32_t kHufQuarterMax = 128;       // stream bits of a quarter of a piece at most
+constexpr uint32_t kFewSequences = 32;         // a block of fewer is run by all lanes alike, of more by the leading ones
+constexpr uint32_t kLongSequence = 512;        // literals or match bytes of a sequence that all lanes copy in either case
 
 enum : int32_t {
   kOk = 0,
@@ -41,6 +46,11 @@ struct FseCell {
   uint16_t base;     // next state = base + (nb bits read)
   uint8_t sym;
   uint8_t nb;
+};
+
+// Repeat offsets (RFC 8878 3.1.2.5), kept from block to block in a frame.
+struct Rep {
+  uint32_t r0, r1, r2;
 };
 
 // Scratch of the table builds (dead before a Huffman decode starts).
@@ -79,6 +89,12 @@ struct ZState {
   uint32_t have_ll, have_ml, have_of; // a table exists for the Repeat mode
   uint32_t val[3];                    // broadcast: results of single-lane work
   int32_t err;                        // broadcast: error of single-lane work
+  struct {                            // from the leading lanes: a long sequence, or (more == 0) the end of them
+    uint64_t op;
+    uint32_t lp, ll, ml, off, more;
+    int32_t err;
+    Rep rep;
+  } seq;
   uint8_t stage[kStageBytes];         // the current compressed block, when it fits
 };
 static_assert(sizeof(ZState) <= 160u * 1024u / 4, "four tasks per CU");
@@ -692,11 +708,6 @@ __host__ __device__ inline int32_t seq_table(const Team& tm, ZState& z, uint32_t
   return (int32_t)used;
 }
 
-// Repeat offsets (RFC 8878 3.1.2.5), kept from block to block in a frame.
-struct Rep {
-  uint32_t r0, r1, r2;
-};
-
 // Output positions are frame-relative inside dst; `frame0` is where the frame
 // starts. Every lane holds the same values.
 struct Out {
@@ -710,20 +721,126 @@ template <class Team>
 __host__ __device__ inline void team_fill(const Team& tm, uint8_t* d, uint8_t v, uint64_t n) {
   for (uint64_t i = tm.lane(); i < n; i += Team::size) d[i] = v;
 }
-template <class Team>
-__host__ __device__ inline void team_copy(const Team& tm, uint8_t* d, const uint8_t* s, uint64_t n) {
-  // d and s do not overlap: four bytes per lane in flight (past the end, the last byte again)
-  for (uint64_t i = tm.lane(); i < n; i += 4 * Team::size) {
+// N lanes copy s[0, n) to d, which it does not overlap: four bytes per lane in
+// flight (past the end, the last byte again).
+template <uint32_t N>
+__host__ __device__ inline void copy_bytes(uint32_t lane, uint8_t* d, const uint8_t* s, uint64_t n) {
+  for (uint64_t i = lane; i < n; i += 4 * N) {
     uint8_t v[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-      const uint64_t j = i + k * Team::size;
+      const uint64_t j = i + k * N;
       v[k] = s[j < n ? j : n - 1];
     }
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k)
-      if (i + k * Team::size < n) d[i + k * Team::size] = v[k];
+      if (i + k * N < n) d[i + k * N] = v[k];
   }
+}
+template <class Team>
+__host__ __device__ inline void team_copy(const Team& tm, uint8_t* d, const uint8_t* s, uint64_t n) {
+  copy_bytes<Team::size>(tm.lane(), d, s, n);
+}
+
+// One sequence at dst + op by N lanes: ll literals from lit, then ml bytes from
+// `off` before them. Match byte i is d[ll - off + i % off]: earlier output, or
+// this sequence's literals (then read from the literal buffer).
+template <uint32_t N>
+__host__ __device__ inline void run_sequence(uint32_t lane, uint8_t* dst, uint64_t op, const uint8_t* lit, uint32_t ll,
+                                             uint32_t ml, uint32_t off) {
+  if (ll > N) copy_bytes<N>(lane, dst + op, lit, ll);
+  else if (lane < ll) dst[op + lane] = lit[lane];
+  const uint64_t from = op + ll - off;
+  if (off >= ml) {
+    for (uint64_t j = lane; j < ml; j += N) {
+      const uint64_t src = from + j;
+      dst[op + ll + j] = src >= op ? lit[src - op] : dst[src];
+    }
+  } else {
+    // j mod off kept incrementally: j grows by N each round (off < ml < 2^32, so
+    // this is 32-bit arithmetic and two divisions per sequence instead of one
+    // 64-bit modulo per byte)
+    const uint32_t step = N % off;
+    uint32_t r = lane % off;
+    for (uint64_t j = lane; j < ml; j += N) {
+      const uint64_t src = from + r;
+      dst[op + ll + j] = src >= op ? lit[src - op] : dst[src];
+      r += step;
+      if (r >= off) r -= off;
+    }
+  }
+}
+
+// The sequences of a block: nseq of them from the bitstream b[pos, n), literals
+// from lit[0, lsize); o.op and lp move on. LEAD: run by the team's leading lanes,
+// who share the long ones with the others (below); else by all lanes alike.
+template <bool LEAD, class Team>
+__host__ __device__ __forceinline__ int32_t run_sequences(const Team& tm, ZState& z, const uint8_t* b, uint64_t n,
+                                                          uint64_t pos, uint32_t nseq, Out& o, Rep& rep,
+                                                          const uint8_t* lit, uint32_t lsize, uint64_t& lp) {
+  BackBits br;
+  if (pos >= n || !br.init(b + pos, n - pos)) return kErrStream;
+  uint32_t sll = br.read(z.ll_log), sof = br.read(z.of_log), sml = br.read(z.ml_log);
+  uint64_t visible = o.op;              // output below this is visible to every lane
+  for (uint32_t i = 0; i < nseq; ++i) {
+    const FseCell cl = z.ll[sll], co = z.of[sof], cm = z.ml[sml];
+    if (co.sym > kOFMax) return kErrStream;
+    const uint32_t ofv = (1u << co.sym) + br.read(co.sym);
+    const uint32_t ml = z.ml_base[cm.sym] + br.read(z.ml_bits[cm.sym]);
+    const uint32_t ll = z.ll_base[cl.sym] + br.read(z.ll_bits[cl.sym]);
+    uint32_t off;
+    if (ofv > 3) {
+      off = ofv - 3;
+      rep.r2 = rep.r1;
+      rep.r1 = rep.r0;
+      rep.r0 = off;
+    } else {                            // a repeat: shifted by one when the literal length is 0
+      const uint32_t r = ofv - 1 + (ll == 0 ? 1u : 0u);
+      if (r == 0) {
+        off = rep.r0;
+      } else {
+        off = r == 1 ? rep.r1 : r == 2 ? rep.r2 : rep.r0 - 1;
+        if (r != 1) rep.r2 = rep.r1;
+        rep.r1 = rep.r0;
+        rep.r0 = off;
+      }
+    }
+    if (i + 1 < nseq) {                 // state updates: literal lengths, match lengths, offsets
+      sll = cl.base + br.read(cl.nb);
+      sml = cm.base + br.read(cm.nb);
+      sof = co.base + br.read(co.nb);
+    }
+    if (br.bits() < 0) return kErrStream;
+    if (lp + ll > lsize) return kErrStream;
+    if (o.op + ll + ml > o.cap) return kErrOutput;
+    if (off == 0 || off > o.op + ll - o.frame0) return kErrOffset;
+    if (LEAD && (ll > kLongSequence || ml > kLongSequence)) {
+      if (tm.lane() == 0) {
+        z.seq.op = o.op;
+        z.seq.lp = (uint32_t)lp;
+        z.seq.ll = ll;
+        z.seq.ml = ml;
+        z.seq.off = off;
+        z.seq.more = 1;
+      }
+      tm.sync();
+      run_sequence<Team::size>(tm.lane(), o.dst, o.op, lit + lp, ll, ml, off);
+      tm.sync();
+      visible = o.op + ll + ml;
+    } else {
+      // a match that reads output above `visible` waits for it first
+      const uint64_t from = o.op + ll - off, reach = from + (off < ml ? off : ml);
+      if ((reach < o.op ? reach : o.op) > visible) {
+        if (LEAD) tm.lead_sync();
+        else tm.sync();
+        visible = o.op;
+      }
+      run_sequence<LEAD ? Team::lead_size : Team::size>(tm.lane(), o.dst, o.op, lit + lp, ll, ml, off);
+    }
+    o.op += ll + ml;
+    lp += ll;
+  }
+  return br.bits() == 0 ? kOk : kErrStream;
 }
 
 // One compressed block b[0, n) (RFC 8878 3.1.1.3). rep: repeat offsets. Literals
@@ -846,76 +963,41 @@ __host__ __device__ __forceinline__ int32_t zstd_block(const Team& tm, ZState& z
       if (used < 0) return kErrTable;
       pos += (uint32_t)used;
     }
-    BackBits br;
-    if (pos >= n || !br.init(b + pos, n - pos)) return kErrStream;
-    uint32_t sll = br.read(z.ll_log), sof = br.read(z.of_log), sml = br.read(z.ml_log);
-    uint64_t visible = o.op;            // every lane's output below this is visible to all
-    for (uint32_t i = 0; i < nseq; ++i) {
-      const FseCell cl = z.ll[sll], co = z.of[sof], cm = z.ml[sml];
-      if (co.sym > kOFMax) return kErrStream;
-      const uint32_t ofv = (1u << co.sym) + br.read(co.sym);
-      const uint32_t ml = z.ml_base[cm.sym] + br.read(z.ml_bits[cm.sym]);
-      const uint32_t ll = z.ll_base[cl.sym] + br.read(z.ll_bits[cl.sym]);
-      uint32_t off;
-      if (ofv > 3) {
-        off = ofv - 3;
-        rep.r2 = rep.r1;
-        rep.r1 = rep.r0;
-        rep.r0 = off;
-      } else {                          // a repeat: shifted by one when the literal length is 0
-        const uint32_t r = ofv - 1 + (ll == 0 ? 1u : 0u);
-        if (r == 0) {
-          off = rep.r0;
-        } else {
-          off = r == 1 ? rep.r1 : r == 2 ? rep.r2 : rep.r0 - 1;
-          if (r != 1) rep.r2 = rep.r1;
-          rep.r1 = rep.r0;
-          rep.r0 = off;
+    // Most sequences of a block of many are a few bytes long, and each waits for its
+    // bits, its table entries and the output it copies from, so more wavefronts
+    // add nothing but a barrier between them and their share of the issue slots:
+    // the leading lanes run them, and the others wait for a long one or the end.
+    // A few sequences among many bytes want every lane, and no hand-over. MI355X, a
+    // frame of 168 KB of text by all lanes / the leading ones 17.3 / 16.5 ms, 768 side
+    // by side 20.8 / 18.8; 65 vectors of 4,096 indices (three or four sequences
+    // each) 46.1 / 48 us.
+    if (Team::size == Team::lead_size || nseq < kFewSequences) {
+      const int32_t e = run_sequences<false>(tm, z, b, n, pos, nseq, o, rep, lit, lsize, lp);
+      if (e) return e;
+    } else {
+      if (tm.leads()) {
+        const int32_t e = run_sequences<true>(tm, z, b, n, pos, nseq, o, rep, lit, lsize, lp);
+        if (tm.lane() == 0) {
+          z.seq.op = o.op;
+          z.seq.lp = (uint32_t)lp;
+          z.seq.err = e;
+          z.seq.more = 0;
+          z.seq.rep = rep;
         }
-      }
-      if (i + 1 < nseq) {               // state updates: literal lengths, match lengths, offsets
-        sll = cl.base + br.read(cl.nb);
-        sml = cm.base + br.read(cm.nb);
-        sof = co.base + br.read(co.nb);
-      }
-      if (br.bits() < 0) return kErrStream;
-      if (lp + ll > lsize) return kErrStream;
-      if (o.op + ll + ml > o.cap) return kErrOutput;
-      if (off == 0 || off > o.op + ll - o.frame0) return kErrOffset;
-      // match byte i is d[ll - off + i % off]: earlier output, or this
-      // sequence's literals (then read from the literal buffer). Output below
-      // `visible` has been written before the last barrier; a match that reads
-      // above it waits for one first.
-      const uint64_t from = o.op + ll - off;
-      const uint64_t reach = from + (off < ml ? off : ml);
-      if ((reach < o.op ? reach : o.op) > visible) {
         tm.sync();
-        visible = o.op;
-      }
-      uint8_t* d = o.dst + o.op;
-      team_copy(tm, d, lit + lp, ll);
-      if (off >= ml) {
-        for (uint64_t j = tm.lane(); j < ml; j += Team::size) {
-          const uint64_t src = from + j;
-          o.dst[o.op + ll + j] = src >= o.op ? lit[lp + (src - o.op)] : o.dst[src];
-        }
       } else {
-        // j mod off kept incrementally: j grows by the team size each round
-        // (off < ml < 2^32, so this is 32-bit arithmetic and two divisions per
-        // sequence instead of one 64-bit modulo per byte)
-        const uint32_t off32 = off, step = Team::size % off32;
-        uint32_t r = tm.lane() % off32;
-        for (uint64_t j = tm.lane(); j < ml; j += Team::size) {
-          const uint64_t src = from + r;
-          o.dst[o.op + ll + j] = src >= o.op ? lit[lp + (src - o.op)] : o.dst[src];
-          r += step;
-          if (r >= off32) r -= off32;
+        for (;;) {
+          tm.sync();
+          if (!z.seq.more) break;
+          run_sequence<Team::size>(tm.lane(), o.dst, z.seq.op, lit + z.seq.lp, z.seq.ll, z.seq.ml, z.seq.off);
+          tm.sync();
         }
       }
-      o.op += ll + ml;
-      lp += ll;
+      if (z.seq.err) return z.seq.err;
+      o.op = z.seq.op;
+      lp = z.seq.lp;
+      rep = z.seq.rep;                  // a later block may be run by all lanes
     }
-    if (br.bits() != 0) return kErrStream;
   }
   if (o.op + (lsize - lp) > o.cap) return kErrOutput;
   team_copy(tm, o.dst + o.op, lit + lp, lsize - lp);

@@ -13,10 +13,11 @@
 // team-parallel decoder of zstd_core.h: tables and the current compressed
 // block (when it is at most 24 KB) in LDS, under 40 KB in all; literals
 // of the current block in LDS too where they fit beside it, else in a 128 KiB
-// slice of the work buffer, matches copied by all lanes. Zstandard is a sequential format (each match may copy bytes
-// of the one before), so a frame is not split across workgroups; the
-// reference's zstd entries are small (norm-weight indices, integer buffers)
-// and many of them go in one launch.
+// slice of the work buffer; a block's many sequences are run by the first
+// wavefront, its few or long ones by all lanes. Zstandard is a sequential format
+// (each match may copy bytes of the one before), so a frame is not split across
+// workgroups; the reference's zstd entries are small (norm-weight indices,
+// integer buffers) and many of them go in one launch.
 //
 // lut_expand_kernel turns lowcard indices into element bytes.
 #include <hip/hip_runtime.h>
@@ -26,6 +27,7 @@
 #include <mutex>
 
 #include "../../include/bigsmall_hip.h"
+#include "lds_limit.h"
 #include "zstd_core.h"
 
 // Work area of bs_zstd_decode_static: BS_ZSTD_STATIC_MAX_TASKS literal slices
@@ -43,10 +45,22 @@ static __device__ __align__(256) uint8_t scratch[(uint64_t)BS_ZSTD_STATIC_MAX_TA
 
 namespace {
 
+constexpr uint32_t kLanes = 256;                       // of a workgroup, which decodes one task
+
+// (A type per kernel below, so that each inlines its decoder: a decoder shared by
+// two kernels is a function called with its state in memory, 10 % slower.)
+template <uint32_t GROUPS>
 struct DevTeam {
-  static constexpr uint32_t size = 256;
+  static constexpr uint32_t size = kLanes;
   __device__ uint32_t lane() const { return threadIdx.x; }
   __device__ void sync() const { __syncthreads(); }
+  static constexpr uint32_t lead_size = 64;            // the first wavefront
+  __device__ bool leads() const { return __builtin_amdgcn_readfirstlane(threadIdx.x / lead_size) == 0; }
+  __device__ void lead_sync() const {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  }
 };
 
 __device__ int32_t status_bits(int32_t e) {
@@ -59,26 +73,41 @@ __device__ int32_t status_bits(int32_t e) {
   }
 }
 
-// Three workgroups per CU: left alone the compiler takes 232 vector registers, which
-// lets in two, at the same speed; 128 registers for four cost the two-chain walks 15 %.
-__global__ __launch_bounds__(256, 3) void zstd_kernel(const bs_zstd_task* __restrict__ tasks, uint8_t* __restrict__ work,
-                                                  uint64_t* __restrict__ out_len, int32_t* __restrict__ status) {
+// GROUPS workgroups per CU (launch, below): left alone the compiler takes 232 vector
+// registers, which lets in two, at the speed of three (166).
+template <uint32_t GROUPS>
+__global__ __launch_bounds__(kLanes, GROUPS) void zstd_kernel(const bs_zstd_task* __restrict__ tasks,
+                                                              uint8_t* __restrict__ work, uint64_t* __restrict__ out_len,
+                                                              int32_t* __restrict__ status) {
   __shared__ bs_zstd::ZState z;
   const bs_zstd_task T = tasks[blockIdx.x];
   uint8_t* lit = work + (uint64_t)blockIdx.x * bs_zstd::kBlockMax;
   uint64_t got = 0;
   int32_t e = bs_zstd::kErrFormat;
   if (T.src && (T.dst || T.dst_len == 0)) {
-    e = bs_zstd::zstd_frames(DevTeam{}, z, T.src, T.src_len, T.dst, T.dst_len, lit, got);
+    e = bs_zstd::zstd_frames(DevTeam<GROUPS>{}, z, T.src, T.src_len, T.dst, T.dst_len, lit, got);
     if (e == bs_zstd::kOk && got != T.dst_len) e = bs_zstd::kErrOutput;
   }
   if (e == bs_zstd::kOk && T.xor_src) {        // a delta: dst ^= base (the frames are all written)
-    for (uint64_t i = threadIdx.x; i < T.dst_len; i += DevTeam::size) T.dst[i] ^= T.xor_src[i];
+    for (uint64_t i = threadIdx.x; i < T.dst_len; i += kLanes) T.dst[i] ^= T.xor_src[i];
   }
   if (threadIdx.x == 0) {
     out_len[blockIdx.x] = e ? 0 : got;
     if (e) atomicOr(status, status_bits(e));
   }
+}
+
+// Up to three tasks per CU run side by side with the registers they like; more take
+// the kernel of 128 registers, four of which fit a CU (as many as its LDS holds),
+// and so end in one round up to four per CU. MI355X, three / four per CU:
+// 1,024 frames of 168 KB of text 35.5 / 19.1 ms, of 4,096 indices 273 / 150 us;
+// below the line 65 vectors of 4,096 indices 53 / 56 us.
+int launch(const bs_zstd_task* tasks, uint32_t n_tasks, uint8_t* work, uint64_t* out_len, int32_t* status, hipStream_t s) {
+  if (n_tasks <= 3ull * bs_internal::device_cus())
+    hipLaunchKernelGGL(zstd_kernel<3>, dim3(n_tasks), dim3(kLanes), 0, s, tasks, work, out_len, status);
+  else
+    hipLaunchKernelGGL(zstd_kernel<4>, dim3(n_tasks), dim3(kLanes), 0, s, tasks, work, out_len, status);
+  return hipGetLastError() == hipSuccess ? BS_OK : BS_ERR_HIP;
 }
 
 // Task blockIdx.y; blockIdx.x strides over its elements.
@@ -135,9 +164,7 @@ int bs_zstd_decode(const bs_zstd_task* d_tasks, uint32_t n_tasks, void* d_work, 
   if (!d_status || (n_tasks && (!d_tasks || !d_work || !d_out_len)) || n_tasks > 0x7FFFFFFFu) return BS_ERR_ARG;
   if (n_tasks == 0) return BS_OK;
   if (work_bytes < bs_zstd_work_bytes(n_tasks)) return BS_ERR_ARG;
-  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(DevTeam::size), 0, (hipStream_t)stream, d_tasks, (uint8_t*)d_work,
-                     d_out_len, d_status);
-  return hipGetLastError() == hipSuccess ? BS_OK : BS_ERR_HIP;
+  return launch(d_tasks, n_tasks, (uint8_t*)d_work, d_out_len, d_status, (hipStream_t)stream);
 }
 
 int bs_zstd_decode_static(const bs_zstd_task* d_tasks, uint32_t n_tasks, uint64_t* d_out_len, int32_t* d_status,
@@ -159,9 +186,7 @@ int bs_zstd_decode_static(const bs_zstd_task* d_tasks, uint32_t n_tasks, uint64_
   // the previous call's launch (on any stream) has finished with the array;
   // an event never recorded is complete
   if (order && hipStreamWaitEvent(s, g_scratch_done[dev], 0) != hipSuccess) return BS_ERR_HIP;
-  hipLaunchKernelGGL(zstd_kernel, dim3(n_tasks), dim3(DevTeam::size), 0, s, d_tasks, (uint8_t*)g_scratch_ptr[dev], d_out_len,
-                     d_status);
-  if (hipGetLastError() != hipSuccess) return BS_ERR_HIP;
+  if (launch(d_tasks, n_tasks, (uint8_t*)g_scratch_ptr[dev], d_out_len, d_status, s) != BS_OK) return BS_ERR_HIP;
   if (order && hipEventRecord(g_scratch_done[dev], s) != hipSuccess) return BS_ERR_HIP;
   return BS_OK;
 }

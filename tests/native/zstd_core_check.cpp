@@ -22,6 +22,7 @@
 #endif
 #include "../../bigsmall_amd/csrc/zstd_core.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -46,6 +47,9 @@ struct OneLane {
   static constexpr uint32_t size = 1;
   uint32_t lane() const { return 0; }
   void sync() const {}
+  static constexpr uint32_t lead_size = 1;
+  bool leads() const { return true; }
+  void lead_sync() const {}
 };
 
 using Bytes = std::vector<uint8_t>;
@@ -77,6 +81,9 @@ struct FiberTeam {
   static constexpr uint32_t size = BS_ZSTD_LANES;
   uint32_t lane() const { return threadIdx.x; }
   void sync() const { __syncthreads(); }
+  static constexpr uint32_t lead_size = 64;           // the first wavefront
+  bool leads() const { return threadIdx.x < lead_size; }
+  void lead_sync() const { __builtin_amdgcn_wave_barrier(); }
 };
 long g_team_mismatch = 0;
 #endif
@@ -161,6 +168,17 @@ int main(int argc, char** argv) {
     std::string s;
     while (s.size() < 300000) s += "the quick brown fox " + std::to_string(rng() % 1000) + " jumps\n";
     data.emplace_back("text", Bytes(s.begin(), s.end()));
+  }
+  {
+    // literal runs and matches of lengths around the line from which all lanes copy
+    Bytes v;
+    for (size_t len : {1ul, 63ul, 64ul, 65ul, 255ul, 1023ul, 1024ul, 1025ul, 1026ul, 4000ul, 30000ul})
+      for (size_t back : {1ul, 7ul, 100ul, 2000ul}) {
+        for (size_t i = 0; i < len; ++i) v.push_back((uint8_t)rng());
+        for (size_t i = 0; i < len + 3; ++i) v.push_back(v[v.size() - std::min(back, v.size())]);
+        v.push_back((uint8_t)rng());
+      }
+    data.insert(data.end() - 1, {"runs", v});
   }
   long round_trips = 0, failures = 0;
   auto expect = [&](const char* what, const Bytes& frame, const Bytes& want) {
