@@ -373,7 +373,9 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
   // Wait states the hardware does not keep itself: two instructions between a
   // vector write of a scalar register and a vector read of it (x: writelane and
   // the next step's readlane of w; w, need, second: the arithmetic), one between
-  // a vector write and a readlane of it (y: s_addc).
+  // a vector write and a readlane of it (y: s_addc). settle() keeps those of the first
+  // step of a run, whose operands the compiler wrote: without it nothing but the
+  // compiler's choice of scalar instructions for them did.
 #ifdef BS_SIMT_CPU
   // every lane finds the slot's symbol in the list by itself (an emulated
   // ballot or readlane costs 64 fiber switches)
@@ -455,7 +457,7 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
   auto settle = [&]() {
     x = uni32(x);
     at = uni32(at);
-    BS_SGPR_SETTLE(x, at);
+    BS_LANE_SETTLE(x, at, win);
   };
   // this lane's step of a batch at i0 out (cnt steps), its exponent into the tile's counts
   auto emit = [&](uint32_t i0, uint32_t cnt) {
@@ -485,6 +487,7 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
       if (at >= kHalf) window();
       settle();
       BS_STEP(0);
+      BS_VGPR_SETTLE(acc);
       const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)acc, 0);
       kept = lane == j ? o : kept;
     }

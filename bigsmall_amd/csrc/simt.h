@@ -16,7 +16,8 @@
 #define BS_KEEP2(a, b) ((void)(a), (void)(b))
 #define BS_KEEP4(a, b, c, d) ((void)(a), (void)(b), (void)(c), (void)(d))
 #define BS_OPAQUE(x) ((void)(x))
-#define BS_SGPR_SETTLE(a, b) ((void)(a), (void)(b))
+#define BS_LANE_SETTLE(x, at, win) ((void)(x), (void)(at), (void)(win))
+#define BS_VGPR_SETTLE(v) ((void)(v))
 #define BS_LDS_ADD(p, v) ((void)atomicAdd((p), (v)))
 #define BS_BFE_U32(dst, x, off, width) ((dst) = ((uint32_t)(x) >> (off)) & ((1u << (width)) - 1u))
 #else
@@ -34,10 +35,13 @@
 #define BS_KEEP4(a, b, c, d) asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d))
 // Hides a value's provenance from the optimiser (it stays in a vector register).
 #define BS_OPAQUE(x) asm volatile("" : "+v"(x))
-// Scalar registers a and b may be read by asm from here on: two wait states pass
-// since a vector instruction (readfirstlane) may have written them (the compiler
-// does not count them for asm).
-#define BS_SGPR_SETTLE(a, b) asm volatile("s_nop 1" : "+s"(a), "+s"(b))
+// Asm that follows may read the scalar registers x and at and the vector register win,
+// at also as a lane select and win by readlane, whatever instruction wrote them: four
+// wait states pass, which is what a lane select needs after a vector instruction (the
+// two others need two and one; the compiler counts none of them into asm).
+#define BS_LANE_SETTLE(x, at, win) asm volatile("s_nop 3" : "+s"(x), "+s"(at), "+v"(win))
+// The vector register v, written last by asm, may be read by a readlane: one wait state.
+#define BS_VGPR_SETTLE(v) asm volatile("s_nop 0" : "+v"(v))
 // dst = bits [off, off + width) of x in one v_bfe_u32 the optimiser cannot
 // rewrite (it turns a field extract followed by a scale into a shift and a
 // mask; kept whole, an LDS address from it is one v_lshl_add). off and width

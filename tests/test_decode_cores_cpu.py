@@ -233,3 +233,39 @@ def test_decode_kernels_optimised_without_instrumentation(tmp_path):
     r = subprocess.run([str(exe), str(cases)], capture_output=True, text=True, timeout=900)
     assert r.returncode == 0, r.stdout + r.stderr[-3000:]
     assert "clean failed 0" in r.stdout.strip().splitlines()[-1]
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_settle_keeps_a_lane_selects_wait_states(tmp_path):
+    """A chain step's asm opens with a readlane whose lane number, source and
+    state the compiler wrote, in whatever way: gfx950 wants four wait states
+    between a vector instruction that writes a scalar register and a readlane
+    that takes its lane number from it, and the compiler counts none into asm.
+    Here all three come from vector instructions (the assembly is built here)."""
+    src = tmp_path / "settle.hip"
+    src.write_text('''#include <stdint.h>
+#include <hip/hip_runtime.h>
+#include "simt.h"
+__global__ void k(const uint32_t* p, uint32_t* o) {
+  uint32_t x = (uint32_t)__builtin_amdgcn_readfirstlane((int)p[threadIdx.x]);
+  uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)p[64 + threadIdx.x]), win = p[128 + threadIdx.x] * 3u, w;
+  BS_LANE_SETTLE(x, at, win);
+  asm volatile("v_readlane_b32 %0, %1, %2" : "=s"(w) : "v"(win), "s"(at));
+  o[threadIdx.x] = w + x;
+}
+''')
+    out = tmp_path / "settle.s"
+    r = subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "--offload-device-only", "-S", "-Xclang",
+                        "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", str(ROOT / "bigsmall_amd" / "csrc"),
+                        str(src), "-o", str(out)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    ops = [l.strip() for l in out.read_text().splitlines() if re.match(r"\s+[sv]_\w+", l)]
+    (use,) = [i for i, l in enumerate(ops) if l.startswith("v_readlane_b32")]
+    w, source, select = re.match(r"v_readlane_b32 (\w+), (\w+), (\w+)", ops[use]).groups()
+    assert any(l.startswith(f"v_readfirstlane_b32 {select},") for l in ops[:use]), ops
+    waits = 0
+    for l in reversed(ops[:use]):                  # wait states back to the last writer of either
+        if re.match(rf"[sv]_\w+ ({source}|{select}),", l):
+            break
+        waits += int(l.split()[1]) + 1 if l.startswith("s_nop") else 1
+    assert waits >= 4, ops
