@@ -235,6 +235,24 @@ def test_decode_kernels_optimised_without_instrumentation(tmp_path):
     assert "clean failed 0" in r.stdout.strip().splitlines()[-1]
 
 
+@pytest.mark.skipif(not Path(CLANG).exists(), reason="needs ROCm's clang++")
+def test_lane_symbol_tables(tmp_path):
+    """The tables by which the GPU's chain steps find their symbol (one or two
+    symbols per lane), which the CPU runs above do not read: every slot belongs
+    to exactly one lane, whose symbol, next state and need of a word are the
+    plain step's (tests/native/lane_syms_check.cpp), with 1 to 128 symbols and
+    one of frequency M among them."""
+    exe = tmp_path / "lane_syms"
+    r = subprocess.run([CLANG, "-std=c++17", "-O2", "-pthread", "-DBS_SIMT_CPU", *SANITIZE, "-I", str(ROOT / "include"),
+                        "-I", str(ROOT / "bigsmall_amd" / "csrc"), "-x", "c++",
+                        str(ROOT / "tests" / "native" / "lane_syms_check.cpp"), "-o", str(exe)],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr[-3000:]
+    assert int(r.stdout.split()[1]) > 700_000
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_settle_keeps_a_lane_selects_wait_states(tmp_path):
     """A chain step's asm opens with a readlane whose lane number, source and

@@ -171,10 +171,9 @@ def test_serial_batch_mixed_formats(gpu):
 
 def test_serial_batch_with_shared_xcd_bins(gpu):
     """Twelve tensors in one batch: more than the eight XCD bins, so bins hold
-    several tensors and only the first of each reads its SE table through the
-    scalar cache (the others from LDS). The layout obeys the bins (every
-    task's SE groups inside one bin, the task array ascending, the grid 8C
-    groups) and every output equals its source."""
+    several tensors. The layout obeys the bins (every task's SE groups inside
+    one bin, the task array ascending, the grid 8C groups), the flags, which have
+    no effect, are zero, and every output equals its source."""
     from bigsmall_amd.codecs import _refstreams
     from bigsmall_amd.device import StatusWord, upload_bytes
     torch = gpu
@@ -200,11 +199,10 @@ def test_serial_batch_with_shared_xcd_bins(gpu):
         g = -(-int(t["n_streams"]) // per)
         assert int(t["se_group_begin"]) // C == (int(t["se_group_begin"]) + g - 1) // C
     bins = begins // C
-    scalar = (tasks["flags"] & _refstreams.FLAG_SE_SCALAR) != 0
     assert len(set(bins.tolist())) == _refstreams.XCD_BINS      # every bin used
-    assert all(scalar[bins == b].sum() <= 1 for b in set(bins.tolist()))
+    assert not tasks["flags"].any()
     st = StatusWord(dev)
-    _say(f"[ref] serial batch of {n} tensors in shared bins, totals {batch.totals}, scalar {int(scalar.sum())}")
+    _say(f"[ref] serial batch of {n} tensors in shared bins, totals {batch.totals}")
     batch.launch(st.ptr, torch.cuda.current_stream(dev).cuda_stream)
     torch.cuda.synchronize()
     st.check("serial batch, shared bins")
