@@ -30,7 +30,8 @@ constexpr uint32_t kStageBytes = 24u << 10;    // compressed blocks up to this s
 constexpr uint32_t kHufGroups = 64;            // pieces of a literal section's streams decoded side by side
 constexpr uint32_t kHufQuarterMax = 128;       // stream bits of a quarter of a piece at most
 constexpr uint32_t kFewSequences = 32;         // a block of fewer is run by all lanes alike, of more by the leading ones
-constexpr uint32_t kLongSequence = 512;        // literals or match bytes of a sequence that all lanes copy in either case
+constexpr uint32_t kLongSequence = 512;        // literals or match bytes from which all lanes copy a sequence in either case
+static_assert((kLongSequence & (kLongSequence - 1)) == 0, "run_sequences tests literals and match bytes together");
 
 enum : int32_t {
   kOk = 0,
@@ -752,7 +753,7 @@ __host__ __device__ inline void run_sequence(uint32_t lane, uint8_t* dst, uint64
   else if (lane < ll) dst[op + lane] = lit[lane];
   const uint64_t from = op + ll - off;
   if (off >= ml) {
-    for (uint64_t j = lane; j < ml; j += N) {
+    for (uint32_t j = lane; j < ml; j += N) {
       const uint64_t src = from + j;
       dst[op + ll + j] = src >= op ? lit[src - op] : dst[src];
     }
@@ -762,7 +763,7 @@ __host__ __device__ inline void run_sequence(uint32_t lane, uint8_t* dst, uint64
     // 64-bit modulo per byte)
     const uint32_t step = N % off;
     uint32_t r = lane % off;
-    for (uint64_t j = lane; j < ml; j += N) {
+    for (uint32_t j = lane; j < ml; j += N) {
       const uint64_t src = from + r;
       dst[op + ll + j] = src >= op ? lit[src - op] : dst[src];
       r += step;
@@ -784,8 +785,8 @@ __host__ __device__ __forceinline__ int32_t run_sequences(const Team& tm, ZState
   uint64_t visible = o.op;              // output below this is visible to every lane
   for (uint32_t i = 0; i < nseq; ++i) {
     const FseCell cl = z.ll[sll], co = z.of[sof], cm = z.ml[sml];
-    if (co.sym > kOFMax) return kErrStream;
-    const uint32_t ofv = (1u << co.sym) + br.read(co.sym);
+    const uint32_t ofc = co.sym & 31u;
+    const uint32_t ofv = (1u << ofc) + br.read(ofc);
     const uint32_t ml = z.ml_base[cm.sym] + br.read(z.ml_bits[cm.sym]);
     const uint32_t ll = z.ll_base[cl.sym] + br.read(z.ll_bits[cl.sym]);
     uint32_t off;
@@ -810,11 +811,14 @@ __host__ __device__ __forceinline__ int32_t run_sequences(const Team& tm, ZState
       sml = cm.base + br.read(cm.nb);
       sof = co.base + br.read(co.nb);
     }
-    if (br.bits() < 0) return kErrStream;
-    if (lp + ll > lsize) return kErrStream;
-    if (o.op + ll + ml > o.cap) return kErrOutput;
-    if (off == 0 || off > o.op + ll - o.frame0) return kErrOffset;
-    if (LEAD && (ll > kLongSequence || ml > kLongSequence)) {
+    // One branch for all that may be wrong: a block of short sequences is bound by
+    // the instructions between two of them, and a branch costs 20 cycles and more.
+    // With 32-bit copy loops, MI355X: consecutive int64 numbers (a sequence per 8
+    // bytes), 300 KB 37.3 -> 35.5 ms, text of 300 KB 30.5 -> 28.8 ms.
+    const bool bad_stream = (co.sym > kOFMax) | (br.bits() < 0) | (lp + ll > lsize);
+    const bool bad_output = o.op + ll + ml > o.cap, bad_offset = (off == 0) | (off > o.op + ll - o.frame0);
+    if (bad_stream | bad_output | bad_offset) return bad_stream ? kErrStream : bad_output ? kErrOutput : kErrOffset;
+    if (LEAD && (ll | ml) >= kLongSequence) {
       if (tm.lane() == 0) {
         z.seq.op = o.op;
         z.seq.lp = (uint32_t)lp;
