@@ -628,3 +628,18 @@ def test_kv_calls_under_a_cuda_default_device_and_on_a_foreign_stream():
     out = cache.get_blocks_multi([(0, [4, 1])], stream=types.SimpleNamespace(cuda_stream=own.cuda_stream))
     for blocks, (b, _) in zip(out[0], want):
         assert torch.equal(blocks, b)
+
+
+def test_kv_requests_of_other_sizes_pin_no_new_memory():
+    """Small requests stage their tables in pinned blocks of one size: after the
+    first of them, one of another table size pins nothing more."""
+    from bigsmall_amd.kv_cache_manager import CompressedKVCache
+    k = (torch.randn(2, 512, 64) * 0.5).to(torch.bfloat16).cuda()
+    cache = CompressedKVCache(device="cuda")
+    cache.set_blocks(0, k, k, block_tokens=16)
+    _say("[kv] requests of 1 to 32 blocks")
+    cache.get_blocks(0, [3])
+    pinned = torch.cuda.host_memory_stats()["num_host_alloc"]
+    for n in (2, 9, 10, 32):
+        cache.get_blocks(0, list(range(n)))
+    assert torch.cuda.host_memory_stats()["num_host_alloc"] == pinned
