@@ -30,7 +30,7 @@ constexpr uint32_t kStageBytes = 24u << 10;    // compressed blocks up to this s
 constexpr uint32_t kHufGroups = 64;            // pieces of a literal section's streams decoded side by side
 constexpr uint32_t kHufQuarterMax = 128;       // stream bits of a quarter of a piece at most
 constexpr uint32_t kFewSequences = 32;         // a block of fewer is run by all lanes alike, of more by the leading ones
-constexpr uint32_t kLongSequence = 512;        // literals or match bytes from which all lanes copy a sequence in either case
+constexpr uint32_t kLongSequence = 128;        // literals or match bytes from which all lanes copy a sequence in either case
 static_assert((kLongSequence & (kLongSequence - 1)) == 0, "run_sequences tests literals and match bytes together");
 
 enum : int32_t {
@@ -974,7 +974,10 @@ __host__ __device__ __forceinline__ int32_t zstd_block(const Team& tm, ZState& z
     // A few sequences among many bytes want every lane, and no hand-over. MI355X, a
     // frame of 168 KB of text by all lanes / the leading ones 17.3 / 16.5 ms, 768 side
     // by side 20.8 / 18.8; 65 vectors of 4,096 indices (three or four sequences
-    // each) 46.1 / 48 us.
+    // each) 46.1 / 48 us. A sequence is long from 128 bytes on, two rounds of the
+    // leading lanes: 4 MB of repeats of 300 bytes 16.9 ms by all lanes alike, 18.3
+    // handed over from 512 bytes, 14.7 from 256 or 128; runs of 200 bytes on average
+    // 24.5, 23.8, 22.7 and 22.2 ms.
     if (Team::size == Team::lead_size || nseq < kFewSequences) {
       const int32_t e = run_sequences<false>(tm, z, b, n, pos, nseq, o, rep, lit, lsize, lp);
       if (e) return e;
