@@ -289,10 +289,10 @@ struct WordWindow {
 // since a chain is serial by its format. Hence no branch in the step (34 cycles
 // taken, 20 not taken, and a renormalisation every sixth step behind it) and no
 // table read (a scalar load through its cache 60 cycles and more, an LDS read 56).
-// MI355X, ns per step with everything around it: 31 with at most 64 symbols (54-57
-// with a table in the scalar cache, 68-77 with one in LDS). A layer of 2048 x 5632
-// in bf16_parallel_v1 5.49 -> 3.48 ms, 4096 x 14336 27.7 -> 17.7 ms, a layer of
-// 512 x 1408 in bf16_se_tans 41.1 -> 22.5 ms (the lane-wise mantissas included).
+// MI355X, ns per step with everything around it: 31 with at most 64 symbols, 45 with
+// up to 128 (54-57 with a table in the scalar cache, 68-77 with one in LDS). A layer of
+// 2048 x 5632 in bf16_parallel_v1 5.62 -> 3.57 ms, 4096 x 14336 28.3 -> 17.7 ms, a layer
+// of 512 x 1408 in bf16_se_tans 44.9 -> 22.6 ms (the lane-wise mantissas included).
 //
 // Renormalisation: the reference loops `while x < L and words remain`. From a
 // state x >= L one decode step leaves x >= 2^4 (SE) or 2^6 (mantissa), so one
@@ -300,6 +300,7 @@ struct WordWindow {
 // and an initial state below L, which no encoder writes, is reported as a
 // corrupt stream. A corrupt stream that runs out of words shifts in its tail
 // word (zero when it has none) and fails the end-of-stream check.
+
 // A symbol of a chain's table in LDS: f | cf << 16, and its output (SE: the
 // word sign<<15 | exp<<7; mantissa: the 7 bits).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -375,7 +376,7 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
   // the next step's readlane of w; w, need, second: the arithmetic), one between
   // a vector write and a readlane of it (y: s_addc). settle() keeps those of the first
   // step of a run, whose operands the compiler wrote: without it nothing but the
-  // compiler's choice of scalar instructions for them did.
+  // compiler's choice of scalar instructions for them did (0.3 % of a chain's time).
 #ifdef BS_SIMT_CPU
   // every lane finds the slot's symbol in the list by itself (an emulated
   // ballot or readlane costs 64 fiber switches)
@@ -504,9 +505,9 @@ __device__ __forceinline__ void serial_chain(const GLB uint8_t* words, uint32_t 
 
 // The SE chain of a tensor with more than 128 live symbols (a checkpoint's weights
 // have 60 or so), of which a lane would hold four or more: each of those costs a
-// step five instructions more in every lane, a table read costs one LDS latency. The table is the task's own, in LDS as 4-byte entries
-// {f | (slot - cf) << 13} beside the slots' output words, shared by the
-// workgroup's chains. The state and the word position stay in vector registers,
+// step five instructions more in every lane, a table read costs one LDS latency.
+// The table is the task's own, in LDS as 4-byte entries {f | (slot - cf) << 13}
+// beside the slots' output words, shared by the workgroup's chains. The state and the word position stay in vector registers,
 // the same in every lane, so that no step waits for a scalar register; the next
 // word comes by ds_bpermute as soon as its position is known, under the next table
 // read; a step's slot goes to its place in the wave's stage, which lane j reads
@@ -579,8 +580,15 @@ __device__ __forceinline__ void table_chain(const GLB uint8_t* words, uint32_t n
 // 64 of them at once from one or two tables in LDS. A step costs more time than a
 // wave-wide chain's (an LDS read on the state's path), but it advances 64
 // chains, so the mantissas take a few wavefronts and leave the issue slots to the
-// SE chains, which set the launch's time. The host lists the buckets table by
-// table; a wavefront whose buckets have more than two tables takes two at a time.
+// SE chains. The host lists the buckets table by table; a wavefront whose buckets
+// have more than two tables takes two at a time.
+//
+// The SE chains set the launch's time where no exponent holds half of a stream, as
+// in weights. A bucket as long as its stream does instead (73 ns a step): MI355X,
+// 8 M elements in 128 streams, ms with a wavefront per bucket and LDS tables / now:
+// normal weights 3.90 / 2.30, one exponent in all 5.80 / 4.78, 90 % one exponent
+// 5.39 / 4.45, values around 1 (two exponents) 3.43 / 2.54; seven such tensors of 1 M
+// elements with one exponent 0.85 / 0.82.
 constexpr uint32_t kLaneRing = 32;                        // words in a lane's ring
 constexpr uint32_t kLaneTables = 2;                       // decode tables of a wavefront
 constexpr uint32_t kLaneB = kLaneTables * 4096 + kLaneRing * 2 * kWave;   // LDS bytes of a wavefront
@@ -782,7 +790,7 @@ __device__ __forceinline__ bs_ref_task pick_task(const bs_ref_task* __restrict__
 // The SE part of the grid has xcd_slots(se_groups) workgroups, a multiple of
 // kXcds: workgroup p serves SE group (p % kXcds) * (slots / kXcds) + p / kXcds
 // (none past the last group). Workgroups go to the XCDs round-robin, so each
-// XCD decodes one contiguous run of groups, which covers one or two tasks.
+// XCD decodes one contiguous run of groups.
 constexpr uint32_t kSerWaves = 4;
 constexpr uint32_t kXcds = 8;
 // A grid part of `count` workgroups dealt to the XCDs in contiguous blocks:
