@@ -471,6 +471,7 @@ class RefBatch:
                 tasks[f][i] = base + off
         buf, _ = _pack(arrays + [tasks.view(np.uint8)])
         self.dev.copy_(torch.from_numpy(buf))
+        self.p_arrays = [base + o for o in offs[:5]]      # of the first task in the array
         self.p_tasks = base + offs[-1]
         self.n_tasks = len(items)
         self.totals = (se_g, mant_g, tile, stream)
@@ -491,7 +492,8 @@ class RefLaunch:
     SERIAL_MIN_UNBOUND elements on, a tensor decodes with one wavefront per
     chain (a one-task bs_refcodec_decode_serial_batch, whose tables are built
     for one output address: pass it here to build them before the first
-    launch); else with one lane per chain (bs_refcodec_decode)."""
+    launch); else, and below SERIAL_MIN_UNBOUND elements to any other address,
+    with one lane per chain (bs_refcodec_decode), which reads the same tables."""
 
     def __init__(self, plan: RefPlan, blob_ptr: int, device, out_ptr: int | None = None):
         import torch
@@ -501,22 +503,25 @@ class RefLaunch:
         self.plan, self.blob_ptr, self.device = plan, blob_ptr, device
         self._batch = None
         self.serial = serial_ok(plan) and (out_ptr is not None or plan.n >= SERIAL_MIN_UNBOUND)
-        if self.serial:
-            if out_ptr is not None:
-                self._batch = (out_ptr, RefBatch([(plan, blob_ptr, out_ptr)], device))
+        if self.serial and out_ptr is not None:
+            self._batch = (out_ptr, RefBatch([(plan, blob_ptr, out_ptr)], device))
+        self.rebind = self.serial and plan.n >= SERIAL_MIN_UNBOUND
+        if self.rebind:
             return
-        buf, offs = _pack(_plan_arrays(plan, blob_ptr))
-        self.dev = torch.from_numpy(buf).to(device)
-        base = self.dev.data_ptr()
-        self.p_streams, self.p_se_table, self.p_bstart, self.p_buckets, self.p_tables = (base + o for o in offs)
+        if self._batch is not None:
+            arrays = self._batch[1].p_arrays
+        else:
+            buf, offs = _pack(_plan_arrays(plan, blob_ptr))
+            self.dev = torch.from_numpy(buf).to(device)
+            arrays = [self.dev.data_ptr() + o for o in offs]
+        self.p_streams, self.p_se_table, self.p_bstart, self.p_buckets, self.p_tables = arrays
         self.perm = torch.empty(max(plan.n, 1), dtype=torch.int32, device=device)
 
     def launch(self, out_ptr: int, status_ptr: int, stream_ptr: int) -> None:
         L = _native.lib()
-        if self.serial:
-            # a one-task batch (its tables built once per output)
-            if self._batch is None or self._batch[0] != out_ptr:
-                self._batch = (out_ptr, RefBatch([(self.plan, self.blob_ptr, out_ptr)], self.device))
+        if self.rebind and (self._batch is None or self._batch[0] != out_ptr):
+            self._batch = (out_ptr, RefBatch([(self.plan, self.blob_ptr, out_ptr)], self.device))   # once per output
+        if self._batch is not None and self._batch[0] == out_ptr:
             self._batch[1].launch(status_ptr, stream_ptr)
             return
         rc = L.bs_refcodec_decode(self.p_streams, self.n_streams, self.p_se_table, self.p_bstart,

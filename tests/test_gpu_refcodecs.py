@@ -328,3 +328,28 @@ def test_small_tensors_on_both_paths(gpu, codec, n):
         torch.cuda.synchronize()
         st.check(codec)
         assert out.cpu().numpy().tobytes() == w.tobytes()
+
+
+@pytest.mark.parametrize("codec", list(CODECS))
+def test_small_tensor_to_an_address_it_was_not_bound_to(gpu, codec):
+    """A small tensor's launch that was given one output address decodes to any
+    other without building or uploading anything (so also while a stream is
+    captured), and to its own again afterwards."""
+    from bigsmall_amd.codecs import _refstreams
+    from bigsmall_amd.device import StatusWord, upload_bytes
+    torch = gpu
+    dev = torch.device("cuda", 0)
+    n = 3000
+    w = _bf16(np.random.default_rng(n).standard_normal(n) * 0.02)
+    blob = CODECS[codec][0](w)
+    d_blob = upload_bytes(blob, dev)
+    outs = [torch.zeros(n, dtype=torch.int16, device=dev) for _ in range(2)]
+    launch = _refstreams.RefLaunch(_refstreams.PARSERS[codec](blob, n), d_blob.data_ptr(), dev, outs[0].data_ptr())
+    batch, st = launch._batch, StatusWord(dev)
+    for out in (outs[1], outs[0], outs[1]):
+        out.zero_()
+        _say(f"[ref] {codec} n={n} to {'its own' if out is outs[0] else 'another'} address")
+        launch.launch(out.data_ptr(), st.ptr, torch.cuda.current_stream(dev).cuda_stream)
+        torch.cuda.synchronize()
+        st.check(codec)
+        assert out.cpu().numpy().tobytes() == w.tobytes() and launch._batch is batch
