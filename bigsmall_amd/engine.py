@@ -312,7 +312,7 @@ class GroupDecoder:
             keep.append(batch)
             batch.launch(status, stream)
         if serial_refs:
-            # every large reference-format tensor of the group in one batched
+            # every reference-format tensor of the group in one batched
             # wave-serial launch: their chains run side by side
             rb = _refstreams.RefBatch(serial_refs, self.device)
             keep.append(rb)
